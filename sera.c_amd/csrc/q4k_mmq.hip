@@ -63,31 +63,26 @@ struct alignas(16) MmqSmem {
      * sits in column c ^ (t & 15), so 16 consecutive tokens reading the same
      * piece hit 16 different bank groups */
     alignas(16) int8_t xs[2][BM][Q4K_QK];
-    /* d8 per [sub-block][token]: the paired tile keeps it as float; the
-     * 32-row tiles keep the fp16 value itself, each 32-token group in the
-     * order of the MFMA result rows a lane holds (token 8q + 4h + i at
-     * 16h + 4q + i), so a lane's 16 scales are one 32-byte run */
-    alignas(16) float d8[PR ? 2 : 1][8][PR ? BM : 4];
-    alignas(16) _Float16 d8h[PR ? 1 : 2][8][PR ? 8 : BM];
+    /* d8 per [sub-block][token] as float; the 32-row tiles keep each
+     * 32-token group in the order of the MFMA result rows a lane holds (token
+     * 8q + 4h + i at 16h + 4q + i), so a lane's 16 scales are one 64-byte run */
+    alignas(16) float d8[2][8][BM];
     alignas(16) _Float16 s8[2][BM][8];       /* fp16 s8, [token][sub-block] */
     alignas(16) _Float16 zero8[8];           /* a zero min-term operand */
 };
 
-/* acc = fma(t, d8, acc) with d8 the low (HI = 0) or high half of a packed
- * fp16 pair: v_fma_mix_f32 converts the half exactly and rounds once, as
- * v_fma_f32 on the converted value would. Written with the accumulator
- * tied to the destination; left to itself the register allocator gives
- * each result a new register and copies the accumulators back per step. */
-template <int HI>
-__device__ __forceinline__ void fma_acc_f16(float &acc, float t, uint32_t d8pair) {
-    if constexpr (HI)
-        asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "+v"(acc) : "v"(t), "v"(d8pair));
-    else
-        asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[0,1,0]" : "+v"(acc) : "v"(t), "v"(d8pair));
+/* A scale that was an fp16 value, kept in a float register: left alone the
+ * compiler folds the conversion into v_fma_mix_f32, which issues at half the
+ * rate of v_fma_f32 once two waves share a SIMD (4.4 against 2.3-2.6 cycles
+ * per instruction measured with two waves; plain fp32 FMAs of the two waves
+ * run side by side, v_fma_mix does not). */
+__device__ __forceinline__ float plain_f32(float v) {
+    asm("" : "+v"(v));
+    return v;
 }
 
-/* Position of token tok in a 32-token group of MmqSmem::d8h. */
-__device__ __forceinline__ int mmq_d8h_pos(int tok) {
+/* Position of row (token or weight row) r in a 32-row group kept in the order of the MFMA result rows. */
+__device__ __forceinline__ int mmq_row_pos(int tok) {
     return (tok & ~31) + 16 * ((tok >> 2) & 1) + 4 * ((tok >> 3) & 3) + (tok & 3);
 }
 
@@ -231,12 +226,7 @@ __device__ __forceinline__ void mmq_segment(
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 union { uint16_t u; _Float16 f; } cv;
-                if constexpr (PR) {
-                    sm.d8[buf][4 * part + e][tok] = h2f_bits(dw[e] & 0xffffu);
-                } else {
-                    cv.u = (uint16_t)(dw[e] & 0xffffu);
-                    sm.d8h[buf][4 * part + e][mmq_d8h_pos(tok)] = cv.f;
-                }
+                sm.d8[buf][4 * part + e][PR ? tok : mmq_row_pos(tok)] = h2f_bits(dw[e] & 0xffffu);
                 cv.u = (uint16_t)(dw[e] >> 16);
                 sm.s8[buf][tok][4 * part + e] = cv.f;
             }
@@ -356,8 +346,8 @@ __device__ __forceinline__ void mmq_segment(
                 for (int nt = 0; nt < 2; nt++) {
                     B0[nt] = unpack_nib(qw[nt][p], h);
                     B1[nt] = unpack_nib(qw[nt][p], 1 - h);
-                    swa[nt] = (float)sw[nt][p].x;
-                    swbb[nt] = (float)sw[nt][p].y;
+                    swa[nt] = plain_f32((float)sw[nt][p].x);
+                    swbb[nt] = plain_f32((float)sw[nt][p].y);
                     nswa[nt] = -SERA_MAGIC_F * swa[nt];
                     nswbb[nt] = -SERA_MAGIC_F * swbb[nt];
                 }
@@ -412,20 +402,24 @@ __device__ __forceinline__ void mmq_segment(
                 }
                 v16i Fn = {};
                 if (i + 1 < NI) Fn = mfma_of(i + 1);
-                const float swb = (float)((b & 1) ? sw[nt][b >> 1].y : sw[nt][b >> 1].x);
+                const float swb = plain_f32((float)((b & 1) ? sw[nt][b >> 1].y : sw[nt][b >> 1].x));
                 const float nswb = -SERA_MAGIC_F * swb;
-                /* the lane's 16 token scales (fp16, exact as float): one
-                 * 32-byte run; v_fma_mix takes each half as it is */
-                const _Float16 *d8p = &sm.d8h[buf][b][BMW * wt + 32 * t + 16 * h];
-                const v4u d8lo = *(const v4u *)d8p, d8hi = *(const v4u *)(d8p + 8);
+                /* The lane's 16 token scales: one 64-byte run. Both FMAs of an
+                 * element are plain fp32 instructions, four of the first kind
+                 * before the four that use them: with two waves per SIMD they
+                 * issue every 2.3-2.6 cycles against 4.4 for v_fma_mix on fp16
+                 * scales (gate/up 25600 x 5120 at 512 tokens 209 -> 197 us,
+                 * 2048 tokens 752 -> 695, down 217 -> 198, same results), for
+                 * four LDS reads per (sub-block, token tile) instead of two. */
+                const float *d8p = &sm.d8[buf][b][BMW * wt + 32 * t + 16 * h];
 #pragma unroll
-                for (int r = 0; r < 16; r += 2) {
-                    const uint32_t pair = r < 8 ? d8lo[r / 2] : d8hi[r / 2 - 4];
-                    float a0 = acc[t][nt][r], a1 = acc[t][nt][r + 1];
-                    fma_acc_f16<0>(a0, scaled_dot(Fc[r], swb, nswb), pair);
-                    fma_acc_f16<1>(a1, scaled_dot(Fc[r + 1], swb, nswb), pair);
-                    acc[t][nt][r] = a0;
-                    acc[t][nt][r + 1] = a1;
+                for (int q = 0; q < 4; q++) {
+                    const v4f d8v = *(const v4f *)(d8p + 4 * q);
+                    float tt[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) tt[e] = scaled_dot(Fc[4 * q + e], swb, nswb);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[t][nt][4 * q + e] = fmaf(tt[e], d8v[e], acc[t][nt][4 * q + e]);
                 }
                 Fc = Fn;
             }
