@@ -184,7 +184,7 @@ int sera_q4k_mmq_streamk(const void *W, const void *mmq_stage, float *Y, float *
                          int M, int N, int K, int wgs, void *stream);
 int sera_q4k_mmq_streamk_wgs(int M);   /* resident workgroups for M tokens (after init) */
 /* Schedule of the MMQ tile kernels for this shape (after init): 2 = whole
- * tiles + split tail (the 64-token tile, M > 32; below), 1 = stream-K
+ * tiles + split tail (M > 32; below), 1 = stream-K
  * (16- and 32-token tiles, M <= 32, from one full round of resident
  * workgroups of tiles), 0 = plain tiles / split-K with the split count of
  * sera_q4k_mmq_splits (a per-CU cost model fitted to MI355X timings); -1
@@ -217,7 +217,8 @@ size_t sera_q4k_mmq_tail_slot_floats(int M, int N, int dp_tiles, int pieces);
  * (mul_mat_q has one kernel family); a dispatch query. */
 int sera_q4k_mmq_uses_fewtok(int M, int N, int K);
 /* MMQ output tiles for M tokens of N rows: 16, 32 or 64 tokens by 256 rows,
- * or 64 by 128 where 256-row tiles would number at most 64. */
+ * or 64 by 128 where 256-row tiles would number at most 64, else 128 by 128
+ * from 65 tokens on. */
 int sera_q4k_mmq_tiles(int M, int N);
 /* Floats of one stream-K or tail slot for M tokens (the largest tile's). */
 int sera_q4k_mmq_slot_floats(int M);

@@ -684,6 +684,467 @@ __global__ __launch_bounds__(256, WPE) void sera_q4k_mmq_tail_kernel(
     mmq_store<TT, WGT, WGN, PR>(y, M, N, m0, n0, acc, accum);
 }
 
+/* ---- wide tile: 128 tokens x 128 rows --------------------------------------- */
+
+/* Prefill tile for more than 64 tokens (sera_mmq_wide): four waves of 128
+ * tokens x 32 rows. Weights are the MFMA's A operand here (result rows =
+ * weight rows) and activations its B operand (a lane owns one token), so
+ *   - a wave unpacks its 32 rows once for four token tiles (the 64 x 256 tile
+ *     unpacks each row for two), and decodes each row's header once, the
+ *     scales in the lanes h = 0 and the mins in the lanes h = 1;
+ *   - d8 is a per-lane scalar, and the row scales reach the lanes that hold
+ *     the result rows through wave-private LDS, 4 reads per sub-block for
+ *     four MFMAs (the token scales of the other tiles take 8 for four).
+ * What bounds it is the fp32 epilogue, 32 FMAs per MFMA (the file comment),
+ * and with two waves ready on each SIMD the card's power: the clock falls to
+ * 1.8-2.0 GHz. So the K loop runs as one pipeline of units (sub-block, token
+ * tile), 8 * TT per super-block, that does not stop at the step's end: region
+ * i issues the MFMA of unit i + 1, one activation load to LDS, the LDS reads
+ * of unit i + 3 and a quarter of the next sub-block's row scales, then runs
+ * the epilogue of unit i; the one barrier of a step comes three units before
+ * its end and waits for loads issued most of a step earlier. Cycles per
+ * launch at 2048 tokens of gate/up (25600 x 5120): 1.66M with the 64 x 256
+ * tile at half-rate FMAs, 1.42M at full rate, 1.25M here; 752 -> 695 -> 675
+ * us. Issuing all activation loads at once costs 5% (the wave waits for the
+ * queue), two waves per SIMD of one 8-wave workgroup was not tried, and
+ * reading the activations three or five units ahead instead of two is within
+ * 1%.
+ *
+ * The last tile of an M that leaves it at most 64 tokens runs as 64 x 128. */
+
+/* LDS of a wide tile, BM = 32 * TT tokens: 80 KB for 128 tokens, half of a
+ * CU's, with no byte to spare for a second workgroup. */
+constexpr int kWideBM = 128, kWideBN = 128;
+template <int TT>
+struct alignas(16) MmqWideSmem {
+    static constexpr int BM = 32 * TT;
+    /* int8 quants of one 256-wide K step, columns swizzled as in MmqSmem */
+    alignas(16) int8_t xs[2][BM][Q4K_QK];
+    alignas(16) float d8[2][8][BM];          /* token scales, [sub-block][token] */
+    alignas(16) _Float16 s8[2][BM][8];       /* fp16 s8, [token][sub-block] */
+    /* each wave's row scales fp16(d*sc_b) of the K step as float: sub-block
+     * b's 32 rows in the order of the MFMA result rows a lane holds (row
+     * 8q + 4h + i at 16h + 4q + i) */
+    alignas(16) float sw[4][8][32];
+};
+
+/* a workgroup barrier after this wave's LDS accesses and all but its VM most
+ * recent vector memory loads (vmcnt counts in order) */
+template <int VM>
+__device__ __forceinline__ void mmq_barrier_vm() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM) : "memory");
+}
+
+/* acc[t] += the tile's sums over super-blocks [kb_begin, kb_end) for token
+ * tiles t < TT; the stage must hold BM rows from m0 on. Ends past a barrier
+ * with no load in flight. */
+template <int TT>
+__device__ __forceinline__ void mmq_wide_segment(MmqWideSmem<TT> &sm, const uint8_t *__restrict__ W,
+                                                 const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
+                                                 int N, int K, int m0, int n0, int kb_begin, int kb_end,
+                                                 v16f (&acc)[4], int tiled) {
+    constexpr int BM = 32 * TT;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, h = lane >> 5;
+    const int nkb = K / Q4K_QK;
+
+    /* this lane's weight row (A operand row l32) */
+    const int row = min(n0 + 32 * wave + l32, N - 1);
+    const uint64_t tbase = q4k_block_offset(tiled, n0, 0, nkb);
+    const uint64_t tend = (uint64_t)N * nkb * Q4K_BLOCK_BYTES - tbase;
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(W + tbase), (short)0, (int)(tend > 0x7fffffffu ? 0x7fffffffu : tend), MMQ_SLOT_RSRC_FLAGS);
+    const uint32_t wvo = (uint32_t)(q4k_block_offset(tiled, row, 0, nkb) - tbase);
+    const uint32_t wvp = wvo + 16u + 16u * h;
+    const int bstride = q4k_block_stride(tiled);
+    auto load_hdr = [&](int kb) -> v4u {
+        return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rw, wvo, kb * bstride, 0));
+    };
+    auto load_piece = [&](int kb, int j) -> v4u {
+        return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rw, wvp + 32u * j, kb * bstride, 0));
+    };
+
+    /* activations: 1 KB (four token rows) per load to LDS; load k of this
+     * wave brings tokens 4 * wave + 16 k .. + 3, columns swizzled */
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t *>(xq + (size_t)m0 * K), (short)0, (int)((uint32_t)BM * (uint32_t)K), MMQ_SLOT_RSRC_FLAGS);
+    const int xt = 4 * wave + (lane >> 4);
+    const uint32_t xvo = (uint32_t)(xt * K + 16 * ((lane & 15) ^ (xt & 15)));
+    auto issue_x = [&](int kb, int buf, int k) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void_t *)&sm.xs[buf][4 * wave + 16 * k][0], 16, xvo,
+                                                 16 * k * K + kb * Q4K_QK, 0, 0);
+    };
+    const int dtok = tid >> 1, dpart = tid & 1;
+    const uint32_t *dsrc = xds + (size_t)(m0 + dtok) * (K / 32) + 4 * dpart;   /* tid < 2 * BM */
+    auto load_d = [&](int kb, v4u &dr) {
+        if (tid < 2 * BM) dr = *(const v4u *)(dsrc + kb * 8);
+    };
+    auto store_d = [&](int buf, const v4u &dr) {
+        if (tid < 2 * BM) {
+            const uint32_t dw[4] = {dr.x, dr.y, dr.z, dr.w};
+            union { uint16_t u[4]; uint2 v; } s;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                sm.d8[buf][4 * dpart + e][dtok] = h2f_bits(dw[e] & 0xffffu);
+                s.u[e] = (uint16_t)(dw[e] >> 16);
+            }
+            *(uint2 *)&sm.s8[buf][dtok][4 * dpart] = s.v;
+        }
+    };
+
+    const v16i magic = magic_seed();
+    const uint32_t hmask = h ? 0xffffffffu : 0u;
+    const int xrow = l32 * Q4K_QK;           /* B operand: token l32 of the tile */
+    const int xswz = l32 & 15;
+    v4u dr = {}, hdr = {}, pw[4] = {}, am = {};
+
+    /* The header's eight scales (lanes h = 0) or negated mins (h = 1) as
+     * fp16 products, one rounding each (q4k_scales_f16). The scales go to the
+     * wave's LDS as float; the mins stay as the min term's A operand, whose k
+     * positions 8..15 (lanes h = 1) carry the eight sub-blocks and whose
+     * others are zero. */
+    auto decode = [&](const v4u hd) {
+        const uint32_t a03 = (h ? hd.z : hd.y);
+        const uint32_t f03 = a03 & 0x3F3F3F3Fu;
+        const uint32_t f47 = ((h ? hd.w >> 4 : hd.w) & 0x0F0F0F0Fu) | ((a03 >> 2) & 0x30303030u);
+        const uint32_t sel = h ? 0x03020302u : 0x01000100u;
+        const h2 mul = as_h2(__builtin_amdgcn_perm(hd.x, hd.x, sel) ^ (h ? 0x80008000u : 0u));
+        const h2 bias = {(_Float16)1024.0f, (_Float16)1024.0f};
+        const h2 p0 = (as_h2(__builtin_amdgcn_perm(0x64646464u, f03, 0x04010400u)) - bias) * mul;
+        const h2 p1 = (as_h2(__builtin_amdgcn_perm(0x64646464u, f03, 0x04030402u)) - bias) * mul;
+        const h2 p2 = (as_h2(__builtin_amdgcn_perm(0x64646464u, f47, 0x04010400u)) - bias) * mul;
+        const h2 p3 = (as_h2(__builtin_amdgcn_perm(0x64646464u, f47, 0x04030402u)) - bias) * mul;
+        if (h == 0) {
+            float *dst = &sm.sw[wave][0][mmq_row_pos(l32)];
+            dst[0] = (float)p0.x;   dst[32] = (float)p0.y;  dst[64] = (float)p1.x;  dst[96] = (float)p1.y;
+            dst[128] = (float)p2.x; dst[160] = (float)p2.y; dst[192] = (float)p3.x; dst[224] = (float)p3.y;
+        }
+        am = (v4u){__builtin_bit_cast(uint32_t, p0) & hmask, __builtin_bit_cast(uint32_t, p1) & hmask,
+                   __builtin_bit_cast(uint32_t, p2) & hmask, __builtin_bit_cast(uint32_t, p3) & hmask};
+    };
+    if (kb_begin < kb_end) {
+#pragma unroll
+        for (int k = 0; k < 2 * TT; k++) issue_x(kb_begin, 0, k);
+        load_d(kb_begin, dr);
+        hdr = load_hdr(kb_begin);
+#pragma unroll
+        for (int j = 0; j < 4; j++) pw[j] = load_piece(kb_begin, j);
+        store_d(0, dr);
+        decode(hdr);
+        hdr = load_hdr(min(kb_begin + 1, kb_end - 1));
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+
+    /* unit i of a step = (sub-block i / TT, token tile i % TT); its
+     * activations and d8 are read PD units before its MFMA into a ring of NB.
+     * BAR: the region that ends a step's reads and begins the next step's. */
+    constexpr int PD = 2, NU = 8 * TT, NB = PD + 1, BAR = NU - PD - 1;
+    load_d(min(kb_begin + 1, kb_end - 1), dr);
+#pragma unroll
+    for (int k = 0; k < NU - 1 - BAR; k++) issue_x(min(kb_begin + 1, kb_end - 1), 1, k);
+    asm volatile("" ::: "memory");
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    auto b_of = [&](int buf, int i) -> v4i {
+        const int b = i / TT, t = i % TT;
+        return *(const v4i *)&sm.xs[buf][0][32 * t * Q4K_QK + xrow + 16 * ((2 * b + h) ^ xswz)];
+    };
+    auto d_of = [&](int buf, int i) -> float { return sm.d8[buf][i / TT][32 * (i % TT) + l32]; };
+    v4f sw[4], swn[4];
+    v4i B[NB];
+    float D[NB];
+#pragma unroll
+    for (int q = 0; q < 4; q++) sw[q] = *(const v4f *)&sm.sw[wave][0][16 * h + 4 * q];
+#pragma unroll
+    for (int i = 0; i < NB; i++) { B[i] = b_of(0, i); D[i] = d_of(0, i); }
+    v4i A = unpack_nib(pw[0], 0);
+    v16i Fc = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B[0], magic, 0, 0, 0);
+    /* (d8, -magic * d8) as a register pair: v_fma_f32 whose second and third
+     * source registers are both even or both odd takes 3.4 instead of 2.06
+     * cycles (two waves per SIMD) */
+    v2f dn = {D[0], -SERA_MAGIC_F * D[0]};
+    asm volatile("" : "+v"(dn));
+    v4u bs = {};
+
+    /* The loop reads one step past its end (LDS only, unused) and loads
+     * clamped steps, so its body has no branch and a fixed count of loads. */
+    for (int kb = kb_begin; kb < kb_end; kb++) {
+        const int buf = (kb - kb_begin) & 1;
+        const int kn = min(kb + 1, kb_end - 1);
+#pragma unroll
+        for (int i = 0; i < NU; i++) {
+            const int b = i / TT, t = i % TT;
+            const int bn = ((i + 1) / TT) & 7;
+            if ((i + 1) % TT == 0) {
+                A = unpack_nib(pw[bn >> 1], bn & 1);
+                if (bn & 1) pw[bn >> 1] = load_piece(kn, bn >> 1);     /* both sub-blocks unpacked */
+            }
+            const v16i Fn = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B[(i + 1) % NB], magic, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            v2f dnn = {D[(i + 1) % NB], -SERA_MAGIC_F * D[(i + 1) % NB]};
+            asm volatile("" : "+v"(dnn));
+            if (i == BAR) {
+                /* this wave's reads of buf are done, and of the loads issued
+                 * since the next step's activations at least three are
+                 * weights (pieces, header): those may still be in flight */
+                store_d(buf ^ 1, dr);
+                mmq_barrier_vm<3>();
+                load_d(min(kb + 2, kb_end - 1), dr);
+            }
+            if (i > BAR && i - BAR - 1 < 2 * TT) {
+                issue_x(min(kb + 2, kb_end - 1), buf, i - BAR - 1);
+                asm volatile("" ::: "memory");
+            } else if (i + NU - BAR - 1 < 2 * TT) {
+                issue_x(kn, buf ^ 1, i + NU - BAR - 1);
+                asm volatile("" ::: "memory");
+            }
+            {
+                const int ip = i + NB;
+                const int bb = ip < NU ? buf : buf ^ 1, ii = ip < NU ? ip : ip - NU;
+                B[i % NB] = b_of(bb, ii);
+                D[i % NB] = d_of(bb, ii);
+            }
+#pragma unroll
+            for (int q = t * (4 / TT); q < (t + 1) * (4 / TT); q++)
+                swn[q] = *(const v4f *)&sm.sw[wave][(b + 1) & 7][16 * h + 4 * q];
+            if (i >= 4 && i < 4 + TT) {
+                const int tm = (i - 4 + TT / 2) % TT;   /* min term of a token tile whose epilogues are TT / 2 units away */
+                const v4u bz = {bs.x & hmask, bs.y & hmask, bs.z & hmask, bs.w & hmask};
+                acc[tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, am), __builtin_bit_cast(v8h, bz),
+                                                                 acc[tm], 0, 0, 0);
+            }
+            if (i >= 3 && i < 3 + TT) bs = *(const v4u *)&sm.s8[buf][32 * ((i - 3 + TT / 2) % TT) + l32][0];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                float tt[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) tt[e] = scaled_dot(Fc[4 * q + e], dn.x, dn.y);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    /* volatile keeps the unit's sums in its region; left to
+                     * itself the compiler collects them and spills */
+                    float a = acc[t][4 * q + e];
+                    asm volatile("v_fmac_f32_e32 %0, %1, %2" : "+v"(a) : "v"(tt[e]), "v"(sw[q][e]));
+                    acc[t][4 * q + e] = a;
+                }
+            }
+            if (i == 7 * TT - 1) {
+                decode(hdr);
+                hdr = load_hdr(min(kb + 2, kb_end - 1));
+            }
+            Fc = Fn;
+            dn = dnn;
+            if (t == TT - 1)
+#pragma unroll
+                for (int q = 0; q < 4; q++) sw[q] = swn[q];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        /* the ring positions continue across steps */
+        if constexpr (NU % NB != 0) {
+            v4i Bt[NB]; float Dt[NB];
+#pragma unroll
+            for (int k = 0; k < NB; k++) { Bt[k] = B[(NU + k) % NB]; Dt[k] = D[(NU + k) % NB]; }
+#pragma unroll
+            for (int k = 0; k < NB; k++) { B[k] = Bt[k]; D[k] = Dt[k]; }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+}
+
+/* One wide tile, 128 tokens or, where the stage holds no more than 64 rows
+ * from m0 on, 64. */
+__device__ __forceinline__ void mmq_wide_tile(MmqWideSmem<4> &sm, const uint8_t *__restrict__ W,
+                                              const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
+                                              int Mpad, int N, int K, int m0, int n0, int kb0, int kb1,
+                                              v16f (&acc)[4], int tiled) {
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+    if (Mpad - m0 > 64)
+        mmq_wide_segment<4>(sm, W, xq, xds, N, K, m0, n0, kb0, kb1, acc, tiled);
+    else
+        mmq_wide_segment<2>(*(MmqWideSmem<2> *)&sm, W, xq, xds, N, K, m0, n0, kb0, kb1, acc, tiled);
+}
+
+/* Store a wide tile: lane (l32, h) holds token m0 + 32 t + l32, rows n0 +
+ * 32 * wave + 8q + 4h + 0..3 (four rows as one 16-byte store where Y's rows
+ * are 16-byte aligned). */
+__device__ __forceinline__ void mmq_wide_store(float *__restrict__ out, int M, int N, int m0, int n0,
+                                               const v16f (&acc)[4], int accum) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int l32 = lane & 31, h = lane >> 5;
+    const bool vec = N % 4 == 0 && ((uintptr_t)out & 15u) == 0;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int m = m0 + 32 * t + l32;
+        if (m >= M) continue;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int n = n0 + 32 * wave + 8 * q + 4 * h;
+            float *dst = out + (size_t)m * N + n;
+            v4f v = {acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+            if (vec) {
+                if (n < N) {
+                    if (accum) v = *(const v4f *)dst + v;
+                    *(v4f *)dst = v;
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < N) dst[e] = accum ? dst[e] + v[e] : v[e];
+            }
+        }
+    }
+}
+
+/* Grid over (tile, K split), as sera_q4k_mmq_kernel. */
+__global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_kernel(
+        const uint8_t *__restrict__ W, const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
+        float *__restrict__ y, float *__restrict__ partial, int M, int Mpad, int N, int K, int kb_per_split, int accum,
+        int tiled) {
+    __shared__ __attribute__((aligned(16))) MmqWideSmem<4> sm;
+    const int ntt = (M + kWideBM - 1) / kWideBM;
+    const int nrt = (N + kWideBN - 1) / kWideBN;
+    const int tile = mmq_tile_of(blockIdx.x, ntt * nrt);
+    const int m0 = (tile % ntt) * kWideBM, n0 = (tile / ntt) * kWideBN;
+    const int kb0 = blockIdx.y * kb_per_split;
+    const int kb1 = min(K / Q4K_QK, kb0 + kb_per_split);
+    v16f acc[4];
+    mmq_wide_tile(sm, W, xq, xds, Mpad, N, K, m0, n0, kb0, kb1, acc, tiled);
+    mmq_wide_store(partial ? partial + (size_t)blockIdx.y * M * N : y, M, N, m0, n0, acc, partial ? 0 : accum);
+}
+
+/* Stream-K over wide tiles: the schedule and hand-off of
+ * sera_q4k_mmq_streamk_kernel. */
+__global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_streamk_kernel(
+        const uint8_t *__restrict__ W, const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
+        float *__restrict__ y, float *__restrict__ slots, int *__restrict__ counters, int M, int Mpad, int N, int K,
+        int accum, int tiled) {
+    constexpr int NACC = 64;
+    __shared__ __attribute__((aligned(16))) MmqWideSmem<4> sm;
+    int &s_last = *(int *)&sm.sw[0][0][0];         /* a segment ends past a barrier */
+    const int tid = threadIdx.x;
+    const int P = gridDim.x;
+    const int w = (blockIdx.x & 7) * (P >> 3) + (blockIdx.x >> 3);
+    const int ntt = (M + kWideBM - 1) / kWideBM;
+    const int nrt = (N + kWideBN - 1) / kWideBN;
+    const int nkb = K / Q4K_QK;
+    const int64_t U = (int64_t)ntt * nrt * nkb;
+    const int64_t myu0 = sk_u0(w, U, P), myu1 = sk_u0(w + 1, U, P);
+    for (int64_t u = myu0; u < myu1;) {
+        const int t = (int)(u / nkb);
+        const int kb0 = (int)(u - (int64_t)t * nkb);
+        const int kb1 = (int)min<int64_t>(nkb, kb0 + (myu1 - u));
+        const int m0 = (t % ntt) * kWideBM, n0 = (t / ntt) * kWideBN;
+        v16f acc[4];
+        mmq_wide_tile(sm, W, xq, xds, Mpad, N, K, m0, n0, kb0, kb1, acc, tiled);
+        if (kb0 == 0 && kb1 == nkb) {
+            mmq_wide_store(y, M, N, m0, n0, acc, accum);
+        } else {
+            const int64_t a = (int64_t)t * nkb;
+            const int c0 = sk_owner(a, U, P), c1 = sk_owner(a + nkb - 1, U, P);
+            float *mine = slots + (size_t)(2 * w + (myu0 <= a ? 1 : 0)) * (NACC * 256);
+#pragma unroll
+            for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    __hip_atomic_store(&mine[(size_t)(tt * 16 + r) * 256 + tid], acc[tt][r], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (tid == 0)
+                s_last = __hip_atomic_fetch_add(&counters[t], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == c1 - c0;
+            __syncthreads();
+            const int last = s_last;
+            __syncthreads();                       /* read before the next tile writes sm */
+            if (last) {
+                if (tid == 0) __hip_atomic_store(&counters[t], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int c = c0; c <= c1; c++) {
+                    const float *src = slots + (size_t)(2 * c + (sk_u0(c, U, P) <= a ? 1 : 0)) * (NACC * 256);
+#pragma unroll
+                    for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            const float v = __hip_atomic_load(&src[(size_t)(tt * 16 + r) * 256 + tid], __ATOMIC_RELAXED,
+                                                              __HIP_MEMORY_SCOPE_AGENT);
+                            acc[tt][r] = c == c0 ? v : acc[tt][r] + v;
+                        }
+                }
+                mmq_wide_store(y, M, N, m0, n0, acc, accum);
+            }
+        }
+        u += kb1 - kb0;
+    }
+}
+
+/* Whole wide tiles, then a split tail: the schedule and hand-off of
+ * sera_q4k_mmq_tail_kernel. */
+__global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_tail_kernel(
+        const uint8_t *__restrict__ W, const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
+        float *__restrict__ y, float *__restrict__ slots, int *__restrict__ counters, int M, int Mpad, int N, int K,
+        int dp_tiles, int pieces, int accum, int tiled) {
+    constexpr int NACC = 64;
+    __shared__ __attribute__((aligned(16))) MmqWideSmem<4> sm;
+    const int tid = threadIdx.x;
+    const int ntt = (M + kWideBM - 1) / kWideBM;
+    const int nrt = (N + kWideBN - 1) / kWideBN;
+    const int ntiles = ntt * nrt;
+    const int nkb = K / Q4K_QK;
+    const int wg = blockIdx.x;
+    int t, piece = 0, kb0 = 0, kb1 = nkb;
+    if (wg < dp_tiles) {
+        t = mmq_tile_of(wg, dp_tiles);
+    } else {
+        const int R = ntiles - dp_tiles;
+        const int L = mmq_tile_of(wg - dp_tiles, R * pieces);
+        piece = L / R;
+        t = dp_tiles + (L - piece * R);
+        kb0 = piece * nkb / pieces;
+        kb1 = (piece + 1) * nkb / pieces;
+    }
+    const int m0 = (t % ntt) * kWideBM, n0 = (t / ntt) * kWideBN;
+    v16f acc[4];
+    mmq_wide_tile(sm, W, xq, xds, Mpad, N, K, m0, n0, kb0, kb1, acc, tiled);
+    if (wg < dp_tiles || pieces == 1) {
+        mmq_wide_store(y, M, N, m0, n0, acc, accum);
+        return;
+    }
+    const int r = t - dp_tiles;
+    constexpr int kChunks = NACC / 4;
+    constexpr int kSlotBytes = NACC * 256 * 4;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        slots + (size_t)r * pieces * (NACC * 256), (short)0, pieces * kSlotBytes, MMQ_SLOT_RSRC_FLAGS);
+#pragma unroll
+    for (int j = 0; j < kChunks; j++) {
+        const int tt = j / 4, q0 = 4 * (j & 3);
+        const v4f v = {acc[tt][q0], acc[tt][q0 + 1], acc[tt][q0 + 2], acc[tt][q0 + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), rs, (j * 256 + tid) * 16,
+                                               piece * kSlotBytes, MMQ_SC1);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    int &s_last = *(int *)&sm.sw[0][0][0];
+    if (tid == 0)
+        s_last = __hip_atomic_fetch_add(&counters[r], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == pieces - 1;
+    __syncthreads();
+    if (!s_last) return;
+    if (tid == 0) __hip_atomic_store(&counters[r], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int p = 0; p < pieces; p++) {
+#pragma unroll
+        for (int j = 0; j < kChunks; j++) {
+            const int tt = j / 4, q0 = 4 * (j & 3);
+            const v4f v = __builtin_bit_cast(
+                v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, (j * 256 + tid) * 16, p * kSlotBytes, MMQ_SC1));
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[tt][q0 + e] = p == 0 ? v[e] : acc[tt][q0 + e] + v[e];
+        }
+    }
+    mmq_wide_store(y, M, N, m0, n0, acc, accum);
+}
+
 /* Sums the split-K partials in split order: y = ((p0 + p1) + p2) + ... */
 __global__ __launch_bounds__(256) void sera_splitk_reduce_kernel(
         const float4 *__restrict__ partial, float4 *__restrict__ y, size_t n4, int splits, int accum) {
@@ -743,6 +1204,23 @@ static int mmq_bn(int M, int N) {
     return 256;
 }
 
+/* Whether M tokens of an N-row matrix run the 128 x 128 wide tile: from 65
+ * tokens wherever the 64-token tile would take 256 rows. On one MI355X, us
+ * against the 64 x 256 tile (both with the tail schedule and full-rate FMAs):
+ * gate/up at 96 / 256 / 512 / 2048 tokens 65.2 / 123.1 / 191.3 / 675 against
+ * 69.9 / 125.0 / 197.8 / 714, down at 512 186.5 against 194.5, o at 256 47.8
+ * against 50.2, q at 512 70.9 against 72.3. The narrow matrices keep the
+ * 64 x 128 tile, which leaves them twice as many tiles. */
+static int mmq_wide(int M, int N) { return M > 64 && mmq_bn(M, N) == 256; }
+
+/* Output tiles of the MMQ grid for M tokens. */
+extern "C" int sera_mmq_tiles(int M, int N) {
+    if (mmq_wide(M, N)) return ((M + kWideBM - 1) / kWideBM) * ((N + kWideBN - 1) / kWideBN);
+    const int bm = sera_mmq_bm(M);
+    const int bn = mmq_bn(M, N);
+    return ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+}
+
 /* Workgroups of the stream-K MMQ kernel one CU keeps resident: two for
  * either tile. The 32-token stream-K kernel is built for 2 waves per SIMD:
  * cut to 3 (168 VGPRs) it spills inside the K loop and measured 20-33%
@@ -765,8 +1243,7 @@ static constexpr int kModelCUs = 256, kMaxSplitWgs = 2048;
 
 extern "C" int sera_mmq_splits(int M, int N, int K) {
     const int bm = sera_mmq_bm(M);
-    const int bn = mmq_bn(M, N);
-    const int tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const int tiles = sera_mmq_tiles(M, N);
     const int nkb = K / Q4K_QK;
     const float tile_scale = bm == 16 ? 0.5f : bm == 32 ? 0.6f : 1.0f;
     int best = 1;
@@ -825,6 +1302,14 @@ extern "C" hipError_t sera_launch_q4k_mmq_acc(uint32_t qtype, const void *W, con
         return launch_mmq_cfg<1, 1, 4, 2, 1>(tiled, w, xq, xds, y, partial, M, N, K, splits, accum, s);
     if (sera_mmq_bm(M) == 32)
         return launch_mmq_cfg<1, 1, 4, 2>(tiled, w, xq, xds, y, partial, M, N, K, splits, accum, s);
+    if (mmq_wide(M, N)) {
+        const int nkb = K / Q4K_QK, per = (nkb + splits - 1) / splits;
+        hipLaunchKernelGGL(sera_q4k_mmq_wide_kernel, dim3(sera_mmq_tiles(M, N), splits), dim3(256), 0, s, w, xq, xds, y,
+                           splits > 1 ? partial : nullptr, M, Mpad, N, K, per, accum, tiled);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || splits == 1) return e;
+        return sera_launch_splitk_reduce_acc(partial, y, (size_t)M * N, splits, accum, s);
+    }
     if (mmq_bn(M, N) == 128)
         return launch_mmq_cfg<1, 2, 2, 2>(tiled, w, xq, xds, y, partial, M, N, K, splits, accum, s);
     return launch_mmq_cfg<2, 1, 4, 2>(tiled, w, xq, xds, y, partial, M, N, K, splits, accum, s);
@@ -832,16 +1317,9 @@ extern "C" hipError_t sera_launch_q4k_mmq_acc(uint32_t qtype, const void *W, con
 
 /* ---- stream-K schedule ---------------------------------------------------- */
 
-/* Output tiles of the MMQ grid for M tokens. */
-extern "C" int sera_mmq_tiles(int M, int N) {
-    const int bm = sera_mmq_bm(M);
-    const int bn = mmq_bn(M, N);
-    return ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-}
-
 /* Floats of one stream-K or tail partial slot: the largest tile's
  * accumulators for M tokens (the paired 16-token tile keeps its 32 MFMA
- * rows); a 128-row tile uses half of its slot. */
+ * rows); a 64 x 128 tile uses half of its slot. */
 extern "C" int sera_mmq_slot_floats(int M) {
     const int bm = sera_mmq_bm(M);
     return (bm < 32 ? 32 : bm) * 256;
@@ -881,6 +1359,11 @@ extern "C" hipError_t sera_launch_q4k_mmq_streamk_acc(uint32_t qtype, const void
         return launch_mmq_streamk_cfg<1, 1, 4, 2, 1>(tiled, w, xq, xds, y, slots, counters, M, N, K, P, accum, s);
     if (sera_mmq_bm(M) == 32)
         return launch_mmq_streamk_cfg<1, 1, 4, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, P, accum, s);
+    if (mmq_wide(M, N)) {
+        hipLaunchKernelGGL(sera_q4k_mmq_wide_streamk_kernel, dim3(P), dim3(256), 0, s, w, xq, xds, y, slots, counters,
+                           M, Mpad, N, K, accum, tiled);
+        return hipGetLastError();
+    }
     if (mmq_bn(M, N) == 128)
         return launch_mmq_streamk_cfg<1, 2, 2, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, P, accum, s);
     return launch_mmq_streamk_cfg<2, 1, 4, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, P, accum, s);
@@ -976,6 +1459,11 @@ extern "C" hipError_t sera_launch_q4k_mmq_tail_acc(uint32_t qtype, const void *W
     if (sera_mmq_bm(M) == 32)
         return launch_mmq_tail_cfg<1, 1, 4, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, dp_tiles, pieces,
                                                 accum, s);
+    if (mmq_wide(M, N)) {
+        hipLaunchKernelGGL(sera_q4k_mmq_wide_tail_kernel, dim3(dp_tiles + (T - dp_tiles) * pieces), dim3(256), 0, s, w,
+                           xq, xds, y, slots, counters, M, Mpad, N, K, dp_tiles, pieces, accum, tiled);
+        return hipGetLastError();
+    }
     if (mmq_bn(M, N) == 128)
         return launch_mmq_tail_cfg<1, 2, 2, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, dp_tiles, pieces,
                                                 accum, s);
