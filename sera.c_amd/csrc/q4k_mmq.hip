@@ -970,33 +970,51 @@ __device__ __forceinline__ void mmq_wide_tile(MmqWideSmem<4> &sm, const uint8_t 
 }
 
 /* Store a wide tile: lane (l32, h) holds token m0 + 32 t + l32, rows n0 +
- * 32 * wave + 8q + 4h + 0..3 (four rows as one 16-byte store where Y's rows
- * are 16-byte aligned). */
-__device__ __forceinline__ void mmq_wide_store(float *__restrict__ out, int M, int N, int m0, int n0,
-                                               const v16f (&acc)[4], int accum) {
+ * 32 * wave + 8q + 4h + 0..3. Where Y's rows are 16-byte aligned those four
+ * rows are one store. Elsewhere each 32 x 32 block goes through wave-private
+ * LDS (the activations' space), so a store instruction writes 32 consecutive
+ * rows of two tokens; as single floats from the lanes that hold them, 6706 x
+ * 512 at 565 tokens took 30.1 us instead of 20.3. Callers that reuse the LDS
+ * pass a barrier first. */
+__device__ __forceinline__ void mmq_wide_store(MmqWideSmem<4> &sm, float *__restrict__ out, int M, int N, int m0,
+                                               int n0, const v16f (&acc)[4], int accum) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l32 = lane & 31, h = lane >> 5;
-    const bool vec = N % 4 == 0 && ((uintptr_t)out & 15u) == 0;
+    if (N % 4 == 0 && ((uintptr_t)out & 15u) == 0) {
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const int m = m0 + 32 * t + l32;
-        if (m >= M) continue;
+        for (int t = 0; t < 4; t++) {
+            const int m = m0 + 32 * t + l32;
+            if (m >= M) continue;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int n = n0 + 32 * wave + 8 * q + 4 * h;
-            float *dst = out + (size_t)m * N + n;
-            v4f v = {acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
-            if (vec) {
-                if (n < N) {
-                    if (accum) v = *(const v4f *)dst + v;
-                    *(v4f *)dst = v;
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (n + e < N) dst[e] = accum ? dst[e] + v[e] : v[e];
+            for (int q = 0; q < 4; q++) {
+                const int n = n0 + 32 * wave + 8 * q + 4 * h;
+                if (n >= N) continue;
+                float *dst = out + (size_t)m * N + n;
+                v4f v = {acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+                if (accum) v = *(const v4f *)dst + v;
+                *(v4f *)dst = v;
             }
         }
+        return;
+    }
+    float *tr = (float *)&sm.xs[0][0][0] + wave * (32 * 33);   /* [token][row], rows padded to 33 */
+    const int n = n0 + 32 * wave + l32;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        if (m0 + 32 * t >= M) break;
+#pragma unroll
+        for (int r = 0; r < 16; r++) tr[l32 * 33 + 8 * (r >> 2) + 4 * h + (r & 3)] = acc[t][r];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int m = m0 + 32 * t + 2 * i + h;
+            const float v = tr[(2 * i + h) * 33 + l32];
+            if (m < M && n < N) {
+                float *dst = out + (size_t)m * N + n;
+                *dst = accum ? *dst + v : v;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -1014,7 +1032,7 @@ __global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_kernel(
     const int kb1 = min(K / Q4K_QK, kb0 + kb_per_split);
     v16f acc[4];
     mmq_wide_tile(sm, W, xq, xds, Mpad, N, K, m0, n0, kb0, kb1, acc, tiled);
-    mmq_wide_store(partial ? partial + (size_t)blockIdx.y * M * N : y, M, N, m0, n0, acc, partial ? 0 : accum);
+    mmq_wide_store(sm, partial ? partial + (size_t)blockIdx.y * M * N : y, M, N, m0, n0, acc, partial ? 0 : accum);
 }
 
 /* Stream-K over wide tiles: the schedule and hand-off of
@@ -1042,7 +1060,7 @@ __global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_streamk_kernel(
         v16f acc[4];
         mmq_wide_tile(sm, W, xq, xds, Mpad, N, K, m0, n0, kb0, kb1, acc, tiled);
         if (kb0 == 0 && kb1 == nkb) {
-            mmq_wide_store(y, M, N, m0, n0, acc, accum);
+            mmq_wide_store(sm, y, M, N, m0, n0, acc, accum);
         } else {
             const int64_t a = (int64_t)t * nkb;
             const int c0 = sk_owner(a, U, P), c1 = sk_owner(a + nkb - 1, U, P);
@@ -1073,25 +1091,36 @@ __global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_streamk_kernel(
                             acc[tt][r] = c == c0 ? v : acc[tt][r] + v;
                         }
                 }
-                mmq_wide_store(y, M, N, m0, n0, acc, accum);
+                mmq_wide_store(sm, y, M, N, m0, n0, acc, accum);
             }
         }
+        __syncthreads();   /* the store may have used the activations' LDS */
         u += kb1 - kb0;
     }
 }
 
+/* Up to four matrices of one K on one activation stage: matrix i holds the
+ * row tiles [end[i - 1], end[i]) of the launch. */
+struct MmqWideGroup {
+    const uint8_t *W[4];
+    float *y[4];
+    int N[4];
+    int end[4];
+};
+
 /* Whole wide tiles, then a split tail: the schedule and hand-off of
- * sera_q4k_mmq_tail_kernel. */
+ * sera_q4k_mmq_tail_kernel, over the tiles of all the group's matrices (one
+ * round of a q/k/v or gate/up group is filled by tiles of all of them, where
+ * separate launches each ended in a partly filled round). */
 __global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_tail_kernel(
-        const uint8_t *__restrict__ W, const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
-        float *__restrict__ y, float *__restrict__ slots, int *__restrict__ counters, int M, int Mpad, int N, int K,
-        int dp_tiles, int pieces, int accum, int tiled) {
+        const MmqWideGroup grp, const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
+        float *__restrict__ slots, int *__restrict__ counters, int M, int Mpad, int K, int dp_tiles, int pieces,
+        int accum, int tiled) {
     constexpr int NACC = 64;
     __shared__ __attribute__((aligned(16))) MmqWideSmem<4> sm;
     const int tid = threadIdx.x;
     const int ntt = (M + kWideBM - 1) / kWideBM;
-    const int nrt = (N + kWideBN - 1) / kWideBN;
-    const int ntiles = ntt * nrt;
+    const int ntiles = ntt * grp.end[3];
     const int nkb = K / Q4K_QK;
     const int wg = blockIdx.x;
     int t, piece = 0, kb0 = 0, kb1 = nkb;
@@ -1105,11 +1134,19 @@ __global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_tail_kernel(
         kb0 = piece * nkb / pieces;
         kb1 = (piece + 1) * nkb / pieces;
     }
-    const int m0 = (t % ntt) * kWideBM, n0 = (t / ntt) * kWideBN;
+    const int rt = t / ntt;
+    int g = 0, rt0 = 0;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        if (rt >= grp.end[i]) { g = i + 1; rt0 = grp.end[i]; }
+    const uint8_t *W = g == 0 ? grp.W[0] : g == 1 ? grp.W[1] : g == 2 ? grp.W[2] : grp.W[3];
+    float *y = g == 0 ? grp.y[0] : g == 1 ? grp.y[1] : g == 2 ? grp.y[2] : grp.y[3];
+    const int N = g == 0 ? grp.N[0] : g == 1 ? grp.N[1] : g == 2 ? grp.N[2] : grp.N[3];
+    const int m0 = (t % ntt) * kWideBM, n0 = (rt - rt0) * kWideBN;
     v16f acc[4];
     mmq_wide_tile(sm, W, xq, xds, Mpad, N, K, m0, n0, kb0, kb1, acc, tiled);
     if (wg < dp_tiles || pieces == 1) {
-        mmq_wide_store(y, M, N, m0, n0, acc, accum);
+        mmq_wide_store(sm, y, M, N, m0, n0, acc, accum);
         return;
     }
     const int r = t - dp_tiles;
@@ -1142,7 +1179,7 @@ __global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_tail_kernel(
             for (int e = 0; e < 4; e++) acc[tt][q0 + e] = p == 0 ? v[e] : acc[tt][q0 + e] + v[e];
         }
     }
-    mmq_wide_store(y, M, N, m0, n0, acc, accum);
+    mmq_wide_store(sm, y, M, N, m0, n0, acc, accum);
 }
 
 /* Sums the split-K partials in split order: y = ((p0 + p1) + p2) + ... */
@@ -1210,8 +1247,11 @@ static int mmq_bn(int M, int N) {
  * gate/up at 96 / 256 / 512 / 2048 tokens 65.2 / 123.1 / 191.3 / 675 against
  * 69.9 / 125.0 / 197.8 / 714, down at 512 186.5 against 194.5, o at 256 47.8
  * against 50.2, q at 512 70.9 against 72.3. The narrow matrices keep the
- * 64 x 128 tile, which leaves them twice as many tiles. */
-static int mmq_wide(int M, int N) { return M > 64 && mmq_bn(M, N) == 256; }
+ * 64 x 128 tile, which leaves them twice as many tiles. Rows of Y that are
+ * not 16-byte aligned keep the 64 x 256 tile: its lanes hold neighbouring
+ * rows, the wide tile's go through LDS, which a short K does not pay for
+ * (6706 x 512 at 565 tokens 17.3 against 20.3 us). */
+static int mmq_wide(int M, int N) { return M > 64 && N % 4 == 0 && mmq_bn(M, N) == 256; }
 
 /* Output tiles of the MMQ grid for M tokens. */
 extern "C" int sera_mmq_tiles(int M, int N) {
@@ -1397,27 +1437,64 @@ static float tail_cost(int64_t dp_rounds, int64_t R, int c, int nkb, int P, int 
     return us;
 }
 
-extern "C" void sera_mmq_tail_plan(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles,
-                                   int *pieces) {
-    const int T = sera_mmq_tiles(M, N);
-    const int nkb = K / Q4K_QK;
+/* The wide tile's rounds model. A full round of P workgroups costs
+ * kWideRoundUs per super-block, a last round kWideLoneUs while it leaves every
+ * CU at most one workgroup and kWidePairUs (rising with the second ones, as
+ * the clock falls) above; a split tile's pieces cost kWideSlotUs each (64 KB
+ * written through and read back, all pieces of a launch together at about 7
+ * TB/s) and kWideSplitUs once. Fitted to a sweep of (whole tiles, pieces) on
+ * 13 shapes of 100-2048 tokens: its pick is within 4% of the fastest on each
+ * (the 64 x 256 tile's constants cost 23% there: gate/up at 256 tokens whole
+ * 102.4 us, in 5 pieces 125.7). */
+static constexpr float kWideRoundUs = 5.4f, kWideLoneUs = 3.25f, kWidePairUs = 4.5f, kWidePairSlopeUs = 0.9f;
+static constexpr float kWideSlotUs = 0.018f, kWideSplitUs = 2.5f;
+
+static float wide_cost(int64_t dp_rounds, int64_t R, int c, int nkb, int P, int C) {
+    const int64_t n = R * c;
+    const int w = (nkb + c - 1) / c;
+    const int64_t full = n / P, rem = n % P;
+    float us = (float)dp_rounds * nkb * kWideRoundUs + (float)full * w * kWideRoundUs;
+    if (rem) us += (float)w * (rem > C ? kWidePairUs + kWidePairSlopeUs * (float)(rem - C) / (float)C : kWideLoneUs);
+    if (c > 1) us += kWideSplitUs + kWideSlotUs * (float)n;
+    return us;
+}
+
+/* (whole tiles, pieces) of T tiles of K; wide: the 128 x 128 tile's model,
+ * else the 64 x 256 one's. */
+static void tail_plan(bool wide, int T, int nkb, int cus, size_t slot_floats, size_t max_slot_floats, int *dp_tiles,
+                      int *pieces) {
     const int C = cus > 0 ? cus : kModelCUs;
     const int P = 2 * C;
     const int rounds = T / P;
+    auto cost = [&](int64_t dp_rounds, int64_t R, int c) {
+        return wide ? wide_cost(dp_rounds, R, c, nkb, P, C) : tail_cost(dp_rounds, R, c, nkb, P, C);
+    };
     int best_dp = T, best_c = 1;
-    float best = tail_cost(rounds, T - (int64_t)rounds * P, 1, nkb, P, C);
+    float best = cost(rounds, T - (int64_t)rounds * P, 1);
     for (int fold = 0; fold <= (rounds > 0 ? 1 : 0); fold++) {
         const int dp = (rounds - fold) * P;
         const int R = T - dp;
         if (R == 0) continue;
         for (int c = 2; c <= (nkb < 16 ? nkb : 16); c++) {
-            if ((size_t)R * c * sera_mmq_slot_floats(M) > max_slot_floats) break;
-            const float us = tail_cost(rounds - fold, R, c, nkb, P, C);
+            if ((size_t)R * c * slot_floats > max_slot_floats) break;
+            const float us = cost(rounds - fold, R, c);
             if (us < best) { best = us; best_dp = dp; best_c = c; }
         }
     }
     *dp_tiles = best_dp;
     *pieces = best_c;
+}
+
+extern "C" void sera_mmq_tail_plan(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles,
+                                   int *pieces) {
+    tail_plan(mmq_wide(M, N), sera_mmq_tiles(M, N), K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles,
+              pieces);
+}
+
+/* The same for the `tiles` wide tiles of a group (sera_mmq_group_tiles). */
+extern "C" void sera_mmq_group_plan(int tiles, int M, int K, int cus, size_t max_slot_floats, int *dp_tiles,
+                                    int *pieces) {
+    tail_plan(true, tiles, K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles, pieces);
 }
 
 /* Floats of the tail schedule's slots and ints of its counters. */
@@ -1434,6 +1511,53 @@ static hipError_t launch_mmq_tail_cfg(int tiled, const uint8_t *W, const int8_t 
     const int grid = dp_tiles + (T - dp_tiles) * pieces;
     hipLaunchKernelGGL((sera_q4k_mmq_tail_kernel<TT, WGT, WGN, WPE, PR>), dim3(grid), dim3(256), 0, s, W, xq, xds, y,
                        slots, counters, M, N, K, dp_tiles, pieces, accum, tiled);
+    return hipGetLastError();
+}
+
+/* Wide tiles of a group of matrices (M > 64), or 0 where the group is better
+ * run matrix by matrix: one matrix, a row count that is no multiple of 4, or
+ * no more than kNarrowTileMax 64 x 256 tiles in all. One launch for the group
+ * against one per matrix (k and v on their own narrow tiles): the linear steps
+ * of a Qwen3-32B layer at 512 tokens 795 -> 739 us on MI355X, with the plan
+ * below. */
+extern "C" int sera_mmq_group_tiles(int M, int count, const int *N) {
+    if (M <= 64 || count < 2 || count > 4) return 0;
+    int64_t narrow = 0, wide = 0;
+    for (int i = 0; i < count; i++) {
+        if (N[i] % 4) return 0;
+        narrow += (int64_t)((M + 63) / 64) * ((N[i] + 255) / 256);
+        wide += (int64_t)((M + kWideBM - 1) / kWideBM) * ((N[i] + kWideBN - 1) / kWideBN);
+    }
+    return narrow > kNarrowTileMax && wide <= 0x7fffffff ? (int)wide : 0;
+}
+
+/* Wide tiles of up to four N[i] x K matrices on one stage, under the tail
+ * schedule (slots: (tiles - dp_tiles) * pieces * sera_mmq_slot_floats(M)
+ * floats; counters: one int per split tile, zero on entry and again on exit). */
+extern "C" hipError_t sera_launch_q4k_mmq_wide_group(uint32_t qtype, int count, const void *const *W, float *const *y,
+                                                     const int *N, const void *stage, float *slots, int *counters,
+                                                     int M, int K, int dp_tiles, int pieces, int accum, hipStream_t s) {
+    const int tiled = qtype == SERA_QTYPE_Q4K_TILED;
+    const int Mpad = sera_mmq_padded_rows(M);
+    const sera_stage_layout L = sera_mmq_stage_layout((size_t)Mpad, (size_t)K);
+    const char *base = (const char *)stage;
+    MmqWideGroup g = {};
+    int end = 0;
+    for (int i = 0; i < 4; i++) {
+        if (i < count) {
+            g.W[i] = (const uint8_t *)W[i];
+            g.y[i] = y[i];
+            g.N[i] = N[i];
+            end += (N[i] + kWideBN - 1) / kWideBN;
+        }
+        g.end[i] = end;
+    }
+    const int T = end * ((M + kWideBM - 1) / kWideBM);
+    if (count < 1 || count > 4 || dp_tiles < 0 || dp_tiles > T || pieces < 1 || pieces > K / Q4K_QK)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(sera_q4k_mmq_wide_tail_kernel, dim3(dp_tiles + (T - dp_tiles) * pieces), dim3(256), 0, s, g,
+                       (const int8_t *)(base + L.qs), (const uint32_t *)(base + L.ds), slots, counters, M, Mpad, K,
+                       dp_tiles, pieces, accum, tiled);
     return hipGetLastError();
 }
 
@@ -1459,11 +1583,9 @@ extern "C" hipError_t sera_launch_q4k_mmq_tail_acc(uint32_t qtype, const void *W
     if (sera_mmq_bm(M) == 32)
         return launch_mmq_tail_cfg<1, 1, 4, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, dp_tiles, pieces,
                                                 accum, s);
-    if (mmq_wide(M, N)) {
-        hipLaunchKernelGGL(sera_q4k_mmq_wide_tail_kernel, dim3(dp_tiles + (T - dp_tiles) * pieces), dim3(256), 0, s, w,
-                           xq, xds, y, slots, counters, M, Mpad, N, K, dp_tiles, pieces, accum, tiled);
-        return hipGetLastError();
-    }
+    if (mmq_wide(M, N))
+        return sera_launch_q4k_mmq_wide_group(qtype, 1, &W, &y, &N, stage, slots, counters, M, K, dp_tiles, pieces,
+                                              accum, s);
     if (mmq_bn(M, N) == 128)
         return launch_mmq_tail_cfg<1, 2, 2, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, dp_tiles, pieces,
                                                 accum, s);

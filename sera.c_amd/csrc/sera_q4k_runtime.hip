@@ -1204,6 +1204,25 @@ extern "C" int sera_linear_group(int count, const void *const *geometries, const
             }
         return 0;
     }
+    /* prefill: the group's wide tiles in one launch, unless two outputs share
+     * memory (their products must then run one after the other) */
+    bool disjoint = true;
+    for (int i = 0; i < count; i++)
+        for (int j = i + 1; j < count; j++)
+            if ((uintptr_t)outputs[i] < (uintptr_t)(outputs[j] + (size_t)M * N[j]) &&
+                (uintptr_t)outputs[j] < (uintptr_t)(outputs[i] + (size_t)M * N[i]))
+                disjoint = false;
+    const int group_tiles = q4 && disjoint && g_counters && g_cus > 0 ? sera_mmq_group_tiles(M, count, N) : 0;
+    if (group_tiles > 0) {
+        int dp, pieces;
+        sera_mmq_group_plan(group_tiles, M, K, g_cus, partial_cap, &dp, &pieces);
+        if (pieces == 1 || group_tiles - dp <= kFewtokCounterBase) {
+            if (sera_launch_q4k_mmq_wide_group(qt, count, weights, outputs, N, g_arena, partial, g_counters, M, K, dp,
+                                               pieces, accum, s) != hipSuccess)
+                return fail(-3, "%s: grouped product launch failed", tag);
+            return 0;
+        }
+    }
     for (int i = 0; i < count; i++) {
         hipError_t e;
         const int n = N[i];

@@ -1,5 +1,5 @@
 """The 128 x 128 MMQ tile (65 tokens and more on matrices of more than 64
-64 x 256 tiles) at the edges of its tiles: a last token tile of at most 64
+64 x 256 tiles, rows a multiple of 4) at the edges of its tiles: a last token tile of at most 64
 tokens, ragged rows, one to three K steps, every schedule, the accumulating
 and the unaligned store, both weight layouts. Exact inputs: every schedule
 must give the dequantized product bit for bit."""
@@ -12,8 +12,8 @@ from test_gpu_exact import assert_bits, dev, exact_inputs, expected, mmq_stage, 
 
 pytestmark = pytest.mark.gpu
 
-# (M, N, K): ragged rows (N % 128, N % 4 != 0: scalar stores) or whole ones
-CASES = [(65, 16401, 256), (128, 8452, 512), (129, 5634, 768), (192, 5632, 768), (193, 4353, 256), (321, 3332, 512)]
+# (M, N, K): ragged rows (N % 128 != 0) or whole ones
+CASES = [(65, 16404, 256), (128, 8452, 512), (129, 5636, 768), (192, 5632, 768), (193, 4356, 256), (321, 3332, 512)]
 
 
 @pytest.mark.parametrize("M,N,K", CASES)
@@ -66,3 +66,78 @@ def test_wide_tile_exact(torch, M, N, K):  # noqa: F811
     torch.cuda.synchronize()
     assert np.array_equal(y.cpu().numpy(), base.cpu().numpy() + ref.astype(np.float32))
     assert float(buf[0]) == -7.0 and float(buf[-1]) == -7.0, "store past Y"
+
+
+@pytest.mark.parametrize("M,Ns,K", [(65, [8192, 512, 260], 512), (200, [4096, 1024, 1024, 132], 768),
+                                    (129, [3000, 3000], 256), (300, [1024, 1024], 2048)])
+def test_group_in_one_launch(torch, M, Ns, K):  # noqa: F811
+    """sera_linear_group over 64 tokens: the matrices' wide tiles in one launch
+    (the last case: too few tiles, matrix by matrix), each product bit for bit,
+    and twice the same output, which must not share a launch."""
+    lin = q3q4.Linear(device=0, max_tokens=512, max_features=8192, max_k=2048)
+    rng = np.random.default_rng(M + sum(Ns))
+    data = [exact_inputs(rng, M, n, K) for n in Ns]
+    X = data[0][1]
+    Ws = [dev(torch, w) for w, _ in data]
+    geos = [q3q4.bind_geometry(12, K, n) for n in Ns]
+    say(f"case group M={M} Ns={Ns} K={K}")
+    ys = [nan_out(torch, M, n) for n in Ns]
+    q3q4.linear_group(geos, Ws, ys, dev(torch, X))
+    torch.cuda.synchronize()
+    refs = [expected(w, X, n, K) for (w, _), n in zip(data, Ns)]
+    for i, (y, ref) in enumerate(zip(ys, refs)):
+        assert_bits(y, ref, f"group[{i}]")
+    y = torch.zeros((M, Ns[0]), device="cuda")
+    q3q4.linear_group([geos[0]] * 2, [Ws[0]] * 2, [y, y], dev(torch, X), flags=q3q4.LIN_ACCUMULATE)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), (2 * refs[0]).astype(np.float32)), "accumulating twice into one output"
+    assert lin.workspace_bytes > 0
+
+
+# M * N % 4 != 0: no split-K, so the tail schedule cuts the tiles along K
+@pytest.mark.parametrize("M,N,K", [(203, 1333, 1792), (41, 1333, 1024), (19, 3001, 2048), (13, 1001, 2304), (65, 77, 256)])
+def test_odd_products_split_by_the_tail(torch, M, N, K):  # noqa: F811
+    L = q3q4.load()
+    lin = q3q4.Linear(device=0, max_tokens=512, max_features=8192, max_k=2560)
+    assert L.sera_q4k_mmq_schedule(M, N, K) == 2
+    rng = np.random.default_rng(M + N + K)
+    W, X = exact_inputs(rng, M, N, K)
+    say(f"case odd product M={M} N={N} K={K} plan {q3q4.mmq_tail_plan(M, N, K)}")
+    y = nan_out(torch, M, N)
+    lin(q3q4.bind_geometry(12, K, N), dev(torch, W), dev(torch, X), y)
+    torch.cuda.synchronize()
+    assert_bits(y, expected(W, X, N, K), "odd product")
+    # and Q6_K, against the oracle
+    W6 = oracle.q6k_weights(rng, N, K)
+    lin(q3q4.bind_geometry(14, K, N), dev(torch, W6), dev(torch, X), y)
+    torch.cuda.synchronize()
+    ref = oracle.linear_reference_q6k(W6, X, N, K)
+    assert float(np.max(np.abs(y.cpu().numpy() - ref))) <= 2e-5 * float(np.sqrt(np.mean(ref * ref)))
+
+
+# RMSNorm on rows of one to five 1024-value pieces, few and many rows (a
+# workgroup takes one piece, several or the whole row): the staged quants are
+# those of the quantizer on the normalized row
+@pytest.mark.parametrize("M,K", [(9, 5120), (300, 5120), (300, 2304), (1030, 1280), (1100, 256), (520, 4864)])
+def test_rmsnorm_quantizer_pieces(torch, M, K):  # noqa: F811
+    lin = q3q4.Linear(device=0, max_tokens=1152, max_features=256, max_k=5120)
+    rng = np.random.default_rng(M + K)
+    H = rng.standard_normal((M, K)).astype(np.float32)
+    gamma = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    rows = np.unique(np.concatenate([[0, M - 1], rng.integers(0, M, 4)]))
+    W = oracle.quantize_q4k((rng.standard_normal((64, K)) * 0.02).astype(np.float32))
+    y = nan_out(torch, M, 64)
+    say(f"case rmsnorm pieces M={M} K={K}")
+    q3q4.linear_group([q3q4.bind_geometry(12, K, 64)], [dev(torch, W)], [y], dev(torch, H), gamma=dev(torch, gamma),
+                      eps=1e-6, flags=q3q4.LIN_RMSNORM)
+    torch.cuda.synchronize()
+    xq, xd, xs = oracle.q8_1_mmq(oracle.rmsnorm_fused_order(H[rows], gamma, 1e-6))
+    ref = oracle.gemm_mmq(W, xq, xd, xs, 64, K)
+    got = y.cpu().numpy()
+    assert np.all(np.isfinite(got))
+    # same quants, fp32 sums in another order (2e-5 * rms as for the other schedules)
+    assert float(np.max(np.abs(got[rows] - ref))) <= 2e-5 * float(np.sqrt(np.mean(ref * ref)))
+    lay = q3q4.mmq_stage_layout(M, K)
+    arena = lin.workspace[256 << 10:].cpu().numpy()        # the stage starts after the counters
+    qs = arena[lay["qs"]:lay["qs"] + M * K].view(np.int8).reshape(M, K)
+    assert np.array_equal(qs[rows], xq)
