@@ -184,7 +184,7 @@ int sera_q4k_mmq_streamk(const void *W, const void *mmq_stage, float *Y, float *
                          int M, int N, int K, int wgs, void *stream);
 int sera_q4k_mmq_streamk_wgs(int M);   /* resident workgroups for M tokens (after init) */
 /* Schedule of the MMQ tile kernels for this shape (after init): 2 = whole
- * tiles + split tail (M > 32; below), 1 = stream-K
+ * tiles + split tail (M > 32, and where M*N is no multiple of 4; below), 1 = stream-K
  * (16- and 32-token tiles, M <= 32, from one full round of resident
  * workgroups of tiles), 0 = plain tiles / split-K with the split count of
  * sera_q4k_mmq_splits (a per-CU cost model fitted to MI355X timings); -1
@@ -204,8 +204,8 @@ int sera_q4k_mmq_schedule(int M, int N, int K);
  * (both may be NULL when pieces == 1 or dp_tiles == tiles). accum != 0 adds
  * the product to Y. sera_q4k_mmq_tail_plan gives the schedule's own choice
  * (after init; slots limited to max_slot_floats, or with 0 to what the
- * attached arena holds after the stage: the plan sera_q4k_dense runs for
- * M > 32). */
+ * attached arena holds after the stage: the plan sera_q4k_dense runs where
+ * sera_q4k_mmq_schedule is 2). */
 int sera_q4k_mmq_tail_qt(uint32_t qtype, const void *W, const void *mmq_stage, float *Y, float *slots, int *counters,
                          int M, int N, int K, int dp_tiles, int pieces, int accum, void *stream);
 int sera_q4k_mmq_tail_plan(int M, int N, int K, size_t max_slot_floats, int *dp_tiles, int *pieces);

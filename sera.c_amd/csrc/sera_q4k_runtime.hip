@@ -421,10 +421,15 @@ bool use_streamk(int M, int N, int K) { return g_counters && streamk_rule(M, N, 
  * 96-128: split-K 22.7-30.3 us against the best tail 24.1-34.3; from 80
  * tiles the tail won: o at 256 tokens 50.6 against 54.4, gate/up at 64
  * 44.1 against 48.8, at 512 215.9 against 232.9, down at 512 206.5 against
- * 217.9). Its counters share the stream-K half of the counter region (the
- * two never run at once; both leave it zero). */
+ * 217.9). It also serves, at any batch (below a full round of 16- or
+ * 32-token tiles), the products whose M*N is no multiple of 4, which split-K's 16-byte reduce cannot: run whole, their few
+ * tiles left most CUs idle (1333 x 1792 at 203 tokens, 44 tiles: 21.7 us
+ * whole, 12 in 4 pieces). Its counters share the stream-K half of the counter
+ * region (the two never run at once; both leave it zero). */
 bool tail_rule(int M, int N) {
-    return g_cus > 0 && sera_mmq_bm(M) == 64 && sera_mmq_tiles(M, N) * 8 > 2 * g_cus;
+    if (g_cus <= 0) return false;
+    if (((size_t)M * N) % 4 != 0) return sera_mmq_bm(M) == 64 || sera_mmq_tiles(M, N) < streamk_wgs(M);
+    return sera_mmq_bm(M) == 64 && sera_mmq_tiles(M, N) * 8 > 2 * g_cus;
 }
 
 struct MmqPlan {
@@ -746,8 +751,16 @@ namespace {
 bool q6k_tail_plan(int M, int N, int K, size_t cap, int *dp, int *pieces) {
     if (!g_counters || g_cus <= 0) return false;
     const int T = sera_q6k_mmq_tiles(M, N, K);
-    const int p = 2 * g_cus / T, nkb = K / Q4K_QK;
-    if (T > kFewtokCounterBase || p < 4 || nkb < 5 * p) return false;
+    int p = 2 * g_cus / T;
+    const int nkb = K / Q4K_QK;
+    if (((size_t)M * N) % 4 != 0) {
+        /* split-K's 16-byte reduce cannot serve these: pieces of at least
+         * two super-blocks, else whole tiles */
+        if (p > nkb / 2) p = nkb / 2;
+        if (T > kFewtokCounterBase || p < 2) return false;
+    } else if (T > kFewtokCounterBase || p < 4 || nkb < 5 * p) {
+        return false;
+    }
     const int pc = p < 63 ? p : 63;
     if (sera_q6k_mmq_tail_slot_floats(M, N, K, 0, pc) > cap) return false;
     *dp = 0;
