@@ -207,8 +207,8 @@ __global__ __launch_bounds__(256) void sera_q8_1_row_kernel(
  * 1024-value pieces of its row. span > 1 only with the RMSNorm producer on
  * many rows, where every workgroup of a row sums the whole row's squares
  * first (the RMSNorm + q/k/v and gate/up groups of a 5120-wide layer: 35 us
- * less of 739 at 512 tokens, 46 of 1356 at 2048). Rows >= M (padding up to the MMQ tile) are
- * written as zeros. */
+ * less of 739 at 512 tokens, 46 of 1356 at 2048). Rows >= M (padding up to
+ * the MMQ tile) are written as zeros. */
 template <int PK>
 __global__ __launch_bounds__(256) void sera_q8_1_mmq_kernel(
         const float *__restrict__ x, sera_producer prod, int M, int K, int span, int8_t *__restrict__ qs,
@@ -251,7 +251,10 @@ __global__ __launch_bounds__(256) void sera_q8_1_mmq_kernel(
 }
 
 /* Q6_K MMQ-layout stage: 16 * quant as fp16 [Mpad][K], fp32 d as
- * [K/256][8][Mpad]; grid = (ceil(K/1024), Mpad); rows >= M are zero.
+ * [K/256][8][Mpad]; grid = (ceil(K / (1024 * span)), Mpad), `span` pieces per
+ * workgroup as in sera_q8_1_mmq_kernel (RMSNorm and two 1024 x 5120 Q6_K
+ * matrices at 2048 tokens 167 -> 148 us, at 200 and 512 tokens no change);
+ * rows >= M are zero.
  * ROW = false: the D4 quantizer (MMQ arithmetic): d_inv = 127/amax,
  *   q = roundf(x*d_inv), d = 1/d_inv in fp32.
  * ROW = true: the row quantizer's values (MMVQ arithmetic, the same as
@@ -259,41 +262,47 @@ __global__ __launch_bounds__(256) void sera_q8_1_mmq_kernel(
  *   kept as fp32(fp16(d)), the d8 the MMVQ formula multiplies by. */
 template <bool ROW, int PK>
 __global__ __launch_bounds__(256) void sera_q8_1_q6k_stage_kernel(
-        const float *__restrict__ x, sera_producer prod, int M, int Mpad, int K, _Float16 *__restrict__ xh,
+        const float *__restrict__ x, sera_producer prod, int M, int Mpad, int K, int span, _Float16 *__restrict__ xh,
         float *__restrict__ d8t) {
     const int row = blockIdx.y;
-    const int k = (blockIdx.x * 256 + threadIdx.x) * 4;
-    const float4 v = q8_produce4_row<PK>(x, prod, row, M, K, k);
-    if (k >= K) return;
-
-    float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-    amax = fmaxf(amax, xor_partner<4>(amax));
-    amax = fmaxf(amax, xor_partner<2>(amax));
-    amax = fmaxf(amax, xor_partner<1>(amax));
-    float q0 = 0.0f, q1 = 0.0f, q2 = 0.0f, q3 = 0.0f, d = 0.0f;
-    if (amax != 0.0f) {
-        if (ROW) {
-            const float dr = amax / 127.0f;
-            q0 = roundf(v.x / dr);
-            q1 = roundf(v.y / dr);
-            q2 = roundf(v.z / dr);
-            q3 = roundf(v.w / dr);
-            d = h2f_bits(f2h_bits(dr));
-        } else {
-            const float d_inv = 127.0f / amax;
-            q0 = roundf(v.x * d_inv);
-            q1 = roundf(v.y * d_inv);
-            q2 = roundf(v.z * d_inv);
-            q3 = roundf(v.w * d_inv);
-            d = 1.0f / d_inv;
+    const int k0 = (blockIdx.x * span * 256 + threadIdx.x) * 4;
+    float inv = 0.0f;
+    float4 v = PK == 1 ? q8_produce4_rms(x, prod, row, M, K, k0, &inv) : q8_produce4_row<PK>(x, prod, row, M, K, k0);
+    for (int k = k0, c = 0; k < K; k += 1024) {
+        float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+        amax = fmaxf(amax, xor_partner<4>(amax));
+        amax = fmaxf(amax, xor_partner<2>(amax));
+        amax = fmaxf(amax, xor_partner<1>(amax));
+        float q0 = 0.0f, q1 = 0.0f, q2 = 0.0f, q3 = 0.0f, d = 0.0f;
+        if (amax != 0.0f) {
+            if (ROW) {
+                const float dr = amax / 127.0f;
+                q0 = roundf(v.x / dr);
+                q1 = roundf(v.y / dr);
+                q2 = roundf(v.z / dr);
+                q3 = roundf(v.w / dr);
+                d = h2f_bits(f2h_bits(dr));
+            } else {
+                const float d_inv = 127.0f / amax;
+                q0 = roundf(v.x * d_inv);
+                q1 = roundf(v.y * d_inv);
+                q2 = roundf(v.z * d_inv);
+                q3 = roundf(v.w * d_inv);
+                d = 1.0f / d_inv;
+            }
+        }
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        /* stored as 16*q: |16q| <= 2032 is exact in fp16 */
+        const h4 hq = {(_Float16)(16.0f * q0), (_Float16)(16.0f * q1), (_Float16)(16.0f * q2), (_Float16)(16.0f * q3)};
+        *(h4 *)(xh + (size_t)row * K + k) = hq;
+        if ((threadIdx.x & 7) == 0)
+            d8t[((size_t)(k >> 8) * 8 + ((k >> 5) & 7)) * Mpad + row] = d;
+        if (PK != 1 || ++c == span) break;
+        if (row < M && k + 1024 < K) {
+            const float4 h = *(const float4 *)(x + (size_t)row * K + k + 1024);
+            v = q8_rms_scale(h, inv, *(const float4 *)(prod.gamma + k + 1024));
         }
     }
-    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-    /* stored as 16*q: |16q| <= 2032 is exact in fp16 */
-    const h4 hq = {(_Float16)(16.0f * q0), (_Float16)(16.0f * q1), (_Float16)(16.0f * q2), (_Float16)(16.0f * q3)};
-    *(h4 *)(xh + (size_t)row * K + k) = hq;
-    if ((threadIdx.x & 7) == 0)
-        d8t[((size_t)(k >> 8) * 8 + ((k >> 5) & 7)) * Mpad + row] = d;
 }
 
 #define Q8_DISPATCH_PK(KIND, ...)                                                                         \
@@ -303,20 +312,31 @@ __global__ __launch_bounds__(256) void sera_q8_1_q6k_stage_kernel(
         default: { constexpr int PK = 0; __VA_ARGS__; } break;                                             \
     }
 
+/* 1024-value pieces of a row per workgroup of the DS4 / Q6_K stage kernels.
+ * RMSNorm: as few workgroups per row as keep about four per CU, since each
+ * sums the whole row's squares; else one piece each. */
+static int q8_piece_span(int kind, int Mpad, int K) {
+    if (kind != 1) return 1;
+    const int pieces = (K + 1023) / 1024, want = (1023 + Mpad) / Mpad;
+    const int per_row = want < pieces ? want : pieces;
+    return (pieces + per_row - 1) / per_row;
+}
+
 /* row_formula = 0: D4 (MMQ) values, 1: row-quantizer (MMVQ) values. */
 extern "C" hipError_t sera_launch_q8_1_q6k_stage_p(const float *x, const sera_producer *prod, int M, int Mpad, int K,
                                                    int row_formula, void *stage, hipStream_t stream) {
     const sera_stage_layout L = sera_q6k_mmq_stage_layout((size_t)Mpad, (size_t)K);
     char *base = (char *)stage;
     const sera_producer p = prod ? *prod : sera_producer{0, nullptr, nullptr, 0.0f};
-    dim3 grid((K + 1023) / 1024, Mpad);
+    const int span = q8_piece_span(p.kind, Mpad, K);
+    dim3 grid((K + 1024 * span - 1) / (1024 * span), Mpad);
     Q8_DISPATCH_PK(p.kind,
         if (row_formula)
             hipLaunchKernelGGL((sera_q8_1_q6k_stage_kernel<true, PK>), grid, dim3(256), 0, stream, x, p, M, Mpad, K,
-                               (_Float16 *)(base + L.qs), (float *)(base + L.ds));
+                               span, (_Float16 *)(base + L.qs), (float *)(base + L.ds));
         else
             hipLaunchKernelGGL((sera_q8_1_q6k_stage_kernel<false, PK>), grid, dim3(256), 0, stream, x, p, M, Mpad,
-                               K, (_Float16 *)(base + L.qs), (float *)(base + L.ds)))
+                               K, span, (_Float16 *)(base + L.qs), (float *)(base + L.ds)))
     return hipGetLastError();
 }
 
@@ -337,12 +357,8 @@ extern "C" hipError_t sera_launch_q8_1_mmq_p(const float *x, const sera_producer
     const sera_stage_layout L = sera_mmq_stage_layout((size_t)Mpad, (size_t)K);
     char *base = (char *)stage;
     const sera_producer p = prod ? *prod : sera_producer{0, nullptr, nullptr, 0.0f};
-    const int pieces = (K + 1023) / 1024;
-    /* RMSNorm: as few workgroups per row as keep about four per CU */
-    int per_row = p.kind == 1 ? (1023 + Mpad) / Mpad : pieces;
-    if (per_row > pieces) per_row = pieces;
-    const int span = (pieces + per_row - 1) / per_row;
-    dim3 grid((pieces + span - 1) / span, Mpad);
+    const int span = q8_piece_span(p.kind, Mpad, K);
+    dim3 grid((K + 1024 * span - 1) / (1024 * span), Mpad);
     Q8_DISPATCH_PK(p.kind,
         hipLaunchKernelGGL((sera_q8_1_mmq_kernel<PK>), grid, dim3(256), 0, stream, x, p, M, K, span,
                            (int8_t *)(base + L.qs), (uint32_t *)(base + L.ds)))

@@ -141,3 +141,26 @@ def test_rmsnorm_quantizer_pieces(torch, M, K):  # noqa: F811
     arena = lin.workspace[256 << 10:].cpu().numpy()        # the stage starts after the counters
     qs = arena[lay["qs"]:lay["qs"] + M * K].view(np.int8).reshape(M, K)
     assert np.array_equal(qs[rows], xq)
+
+
+# the Q6_K stage takes the same pieces
+@pytest.mark.parametrize("M,K", [(9, 5120), (300, 2304), (1030, 1280), (1100, 256), (520, 4864)])
+def test_rmsnorm_q6k_stage_pieces(torch, M, K):  # noqa: F811
+    lin = q3q4.Linear(device=0, max_tokens=1152, max_features=256, max_k=5120)
+    rng = np.random.default_rng(M * 2 + K)
+    H = rng.standard_normal((M, K)).astype(np.float32)
+    gamma = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    rows = np.unique(np.concatenate([[0, M - 1], rng.integers(0, M, 4)]))
+    y = nan_out(torch, M, 64)
+    say(f"case rmsnorm Q6_K pieces M={M} K={K}")
+    q3q4.linear_group([q3q4.bind_geometry(14, K, 64)], [dev(torch, oracle.q6k_weights(rng, 64, K))], [y], dev(torch, H),
+                      gamma=dev(torch, gamma), eps=1e-6, flags=q3q4.LIN_RMSNORM)
+    torch.cuda.synchronize()
+    assert np.all(np.isfinite(y.cpu().numpy()))
+    xq, xd = oracle.q8_1_mmq_d4(oracle.rmsnorm_fused_order(H[rows], gamma, 1e-6))
+    lay = q3q4.q6k_mmq_stage_layout(M, K)
+    arena = lin.workspace[256 << 10:].cpu().numpy()        # the stage starts after the counters
+    xh = arena[lay["qs"]:lay["qs"] + 2 * M * K].view(np.float16).reshape(M, K)
+    assert np.array_equal(xh[rows], 16.0 * xq.astype(np.float32))
+    d = arena[lay["d"]:lay["d"] + lay["rows"] * K // 32 * 4].view(np.float32).reshape(K // 32, lay["rows"])
+    assert np.array_equal(d[:, rows].T, np.asarray(xd).reshape(len(rows), K // 32))
