@@ -28,7 +28,10 @@
  *     to fp32 first (relative error at most 2^-24 per term) and then
  *     accumulated, so per-term results do not follow the reference's single
  *     rounding; they are exact whenever I * sw fits 24 bits (integer-exact
- *     inputs), and otherwise differ by about 2^-24 of the term.
+ *     inputs), and otherwise differ by about 2^-24 of the term. The 128 x 128
+ *     tile takes the two scales in the other order, t = I * d8 and acc =
+ *     fma(t, sw, acc): as many roundings, and for scales beyond fp16's range
+ *     what mmq_wide_overflow says.
  *   - the min term is a plain matrix product over the sub-block index,
  *     [tokens x 8] fp16 s8 times [8 x rows] fp16(-dmin*m_b), done once per
  *     super-block by one v_mfma_f32_32x32x16_f16 accumulating into the same
@@ -735,6 +738,65 @@ __device__ __forceinline__ void mmq_barrier_vm() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM) : "memory");
 }
 
+/* The token scale comes first here, fma(F, d8, -1.5 * 2^23 * d8), so a scale
+ * that overflowed fp16 (a block with |x| above about 8.3e6) makes every row of
+ * its token NaN, where the formula and the other tiles, (I * sw) * d8, give
+ * +-inf (NaN only for a zero dot or zero scale, or opposite infinities). acc's
+ * tokens with such a scale in the K range are computed again in that order,
+ * row by row: slow, but reached by NaN only, so elsewhere it costs four
+ * comparisons per tile (25600 x 5120 at 512 tokens 189.0 us without, 188.8
+ * with; down 189.2 and 187.7). A row scale fp16(d * sc) beyond the range gives
+ * +-inf here, as the formula does, and NaN on the other tiles. */
+template <int TT>
+__device__ __forceinline__ void mmq_wide_overflow(const uint8_t *__restrict__ W, const int8_t *__restrict__ xq,
+                                                  const uint32_t *__restrict__ xds, int N, int K, int m0, int n0,
+                                                  int kb_begin, int kb_end, v16f (&acc)[4], int tiled) {
+    bool nan = false;
+#pragma unroll
+    for (int t = 0; t < TT; t++) nan = nan || acc[t][0] != acc[t][0];
+    if (__builtin_amdgcn_ballot_w64(nan) == 0) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int l32 = lane & 31, h = lane >> 5;
+    const int nkb = K / Q4K_QK;
+#pragma unroll 1
+    for (int t = 0; t < TT; t++) {
+        const size_t m = (size_t)(m0 + 32 * t + l32);          /* a staged row: the tile's tokens all are */
+        bool over = false;
+#pragma unroll 1
+        for (int j = kb_begin * 8; j < kb_end * 8; j++) over = over || (xds[m * (K / 32) + j] & 0x7fffu) == 0x7c00u;
+        if (__builtin_amdgcn_ballot_w64(over) == 0) continue;
+#pragma unroll 1
+        for (int r = 0; r < 16; r++) {
+            const int n = min(n0 + 32 * wave + 8 * (r >> 2) + 4 * h + (r & 3), N - 1);
+            float v = 0.0f;
+#pragma unroll 1
+            for (int kb = kb_begin; kb < kb_end; kb++) {
+                const uint8_t *blk = W + q4k_block_offset(tiled, n, kb, nkb);
+                h2 sw[4], mw[4];
+                q4k_scales_f16(*(const v4u *)blk, sw, mw);
+#pragma unroll
+                for (int b = 0; b < 8; b++) {
+                    const uint32_t *q = (const uint32_t *)(blk + 16 + 32 * (b >> 1));
+                    const int *x = (const int *)(xq + m * K + kb * Q4K_QK + 32 * b);
+                    int dot = SERA_MAGIC_BITS;
+#pragma unroll 1
+                    for (int i = 0; i < 8; i++)
+                        dot = __builtin_amdgcn_sdot4((int)((q[i] >> 4 * (b & 1)) & 0x0F0F0F0Fu), x[i], dot, false);
+                    const uint32_t ds = xds[m * (K / 32) + kb * 8 + b];
+                    const float s = (float)((b & 1) ? sw[b >> 1].y : sw[b >> 1].x);
+                    v = fmaf(scaled_dot(dot, s, -SERA_MAGIC_F * s), h2f_bits(ds & 0xffffu), v);
+                    v = fmaf((float)((b & 1) ? mw[b >> 1].y : mw[b >> 1].x), h2f_bits(ds >> 16), v);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < TT; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    if (over && i == t && e == r) acc[i][e] = v;
+        }
+    }
+}
+
 /* acc[t] += the tile's sums over super-blocks [kb_begin, kb_end) for token
  * tiles t < TT; the stage must hold BM rows from m0 on. Ends past a barrier
  * with no load in flight. */
@@ -950,6 +1012,7 @@ __device__ __forceinline__ void mmq_wide_segment(MmqWideSmem<TT> &sm, const uint
         }
     }
     __builtin_amdgcn_s_waitcnt(0);
+    mmq_wide_overflow<TT>(W, xq, xds, N, K, m0, n0, kb_begin, kb_end, acc, tiled);
     __syncthreads();
 }
 

@@ -164,3 +164,27 @@ def test_rmsnorm_q6k_stage_pieces(torch, M, K):  # noqa: F811
     assert np.array_equal(xh[rows], 16.0 * xq.astype(np.float32))
     d = arena[lay["d"]:lay["d"] + lay["rows"] * K // 32 * 4].view(np.float32).reshape(K // 32, lay["rows"])
     assert np.array_equal(d[:, rows].T, np.asarray(xd).reshape(len(rows), K // 32))
+
+
+# |x| above 8.3e6 overflows the fp16 token scale: the formula's (I * sw) * inf is +-inf, and NaN only where the dot or the
+# scale is zero or infinities of both signs meet. M = 193: both token-tile bodies; the last token's second block overflows too.
+@pytest.mark.parametrize("dp,pieces", [(10 ** 6, 1), (0, 2)])
+def test_wide_tile_token_scale_overflow(torch, dp, pieces):  # noqa: F811
+    M, N, K = 193, 4356, 512
+    tiles = q3q4.load().sera_q4k_mmq_tiles(M, N)
+    rng = np.random.default_rng(5)
+    W, X = exact_inputs(rng, M, N, K)
+    signs = np.repeat([1.0, -1.0], 16).astype(np.float32)       # a zero sum keeps the min term finite
+    for m, b in ((3, 0), (77, 9), (127, 15), (128, 4), (192, 2), (192, 12)):
+        X[m, 32 * b:32 * b + 32] = 1e7 * rng.permutation(signs)
+    xq, xd, xs = oracle.q8_1_mmq(X)
+    ref = oracle.gemm_mmq(W, xq, xd, xs, N, K)
+    lost = np.isinf(ref)
+    assert lost.sum() > 2 * N and np.isnan(ref).any() and np.isfinite(ref).sum() == (M - 5) * N
+    say(f"case wide scale overflow M={M} N={N} K={K} dp_tiles={min(dp, tiles)} pieces={pieces}")
+    slots = torch.empty(max(q3q4.mmq_tail_slot_floats(M, N, min(dp, tiles), pieces), 1), dtype=torch.float32, device="cuda")
+    counters = torch.zeros(tiles, dtype=torch.int32, device="cuda")
+    y = nan_out(torch, M, N)
+    q3q4.mmq_tail(dev(torch, W), mmq_stage(torch, X), y, M, N, K, min(dp, tiles), pieces, slots=slots, counters=counters)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy().astype(np.float64), ref, equal_nan=True)
