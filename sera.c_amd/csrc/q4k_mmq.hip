@@ -1474,73 +1474,47 @@ extern "C" hipError_t sera_launch_q4k_mmq_streamk_acc(uint32_t qtype, const void
 
 /* ---- whole tiles + split tail ---------------------------------------------- */
 
-/* Whole-tile workgroups and K pieces of the tail schedule for M tokens of an
- * N x K matrix on `cus` compute units (64-token tiles, M > 32). The device
- * keeps 2 workgroups per CU resident, so P = 2 * cus run per round. The
- * whole tiles are a multiple of P (all full rounds, or one round fewer);
- * the R tiles left are cut into c K ranges (c = 1: whole as well). Each
- * choice is priced by a rounds model of the greedy dispatch: rounds of P
- * workgroups at kTailPairUs per super-block, a last partial round at
- * kTailLoneUs when it fills no more than one workgroup per CU, and
- * kTailFixUs per piece of a split tile (the hand-off and the last piece's
- * reads). Fitted to a sweep of (whole tiles, c) on 14 Qwen3-32B shapes
- * (q, k/v, o, gate/up, down at 64-2048 tokens) on MI355X: its pick is
- * within 1.6% of the fastest measured choice on every shape where the
- * schedule is used (sera_q4k_mmq_schedule). The split tiles' slots must
- * fit max_slot_floats. */
-static constexpr float kTailPairUs = 5.0f, kTailLoneUs = 3.2f, kTailFixUs = 1.5f;
+/* Fitted on MI355X to the kernel's times under every (whole tiles, pieces) of
+ * random shapes; what the pick costs over the fastest of them:
+ *   16 x 256 tile, 109 shapes of 9-16 tokens: 0.6%, at most 11%;
+ *   32 x 256 and 64 x 128 tiles (as many outputs to a workgroup), 126 and 347
+ *     shapes of 17-1024 tokens: 0.6% and 0.9%, at most 8% and 20%. The 64 x
+ *     256 tile's constants cost these three 3-5%, at most 37%, above all by
+ *     splitting a short K that runs faster whole (15767 x 768 at 11 tokens:
+ *     62 whole tiles 10.7 us a call, in 3 pieces 11.9);
+ *   64 x 256 tile: 14 Qwen3-32B shapes (q, k/v, o, gate/up, down at 64-2048
+ *     tokens), at most 1.6%;
+ *   128 x 128 tile: 13 shapes of 100-2048 tokens, at most 4%. */
+static constexpr sera_tile_cost kCost16 = {3.1f, 0.0f, 2.17f, 2.25f, 2.9f, 0.021f, 1.35f, 0.37f, 2.25f};
+static constexpr sera_tile_cost kCost8192 = {2.9f, 1.7f, 2.55f, 3.05f, 3.5f, 0.018f, 1.0f, 0.44f, 3.05f};
+static constexpr sera_tile_cost kCost64x256 = {5.0f, 0.0f, 3.2f, 0.0f, 5.0f, 0.0f, 0.0f, 1.5f, 0.0f};
+static constexpr sera_tile_cost kCostWide = {5.4f, 0.0f, 3.25f, 0.0f, 4.5f, 0.018f, 2.5f, 0.0f, 0.0f};
 
-static float tail_cost(int64_t dp_rounds, int64_t R, int c, int nkb, int P, int C) {
-    const int64_t n = R * c;
-    const int w = (nkb + c - 1) / c;
-    const int64_t full = n / P, rem = n % P;
-    float us = (float)dp_rounds * nkb * kTailPairUs + (float)full * w * kTailPairUs;
-    if (rem) us += (float)w * (rem > C ? kTailPairUs : kTailLoneUs);
-    if (c > 1) us += kTailFixUs * c;
-    return us;
+static const sera_tile_cost &tile_cost(int M, int N) {
+    if (mmq_wide(M, N)) return kCostWide;
+    if (sera_mmq_bm(M) == 16) return kCost16;
+    return sera_mmq_bm(M) == 32 || mmq_bn(M, N) == 128 ? kCost8192 : kCost64x256;
 }
 
-/* The wide tile's rounds model. A full round of P workgroups costs
- * kWideRoundUs per super-block, a last round kWideLoneUs while it leaves every
- * CU at most one workgroup and kWidePairUs (rising with the second ones, as
- * the clock falls) above; a split tile's pieces cost kWideSlotUs each (64 KB
- * written through and read back, all pieces of a launch together at about 7
- * TB/s) and kWideSplitUs once. Fitted to a sweep of (whole tiles, pieces) on
- * 13 shapes of 100-2048 tokens: its pick is within 4% of the fastest on each
- * (the 64 x 256 tile's constants cost 23% there: gate/up at 256 tokens whole
- * 102.4 us, in 5 pieces 125.7). */
-static constexpr float kWideRoundUs = 5.4f, kWideLoneUs = 3.25f, kWidePairUs = 4.5f, kWidePairSlopeUs = 0.9f;
-static constexpr float kWideSlotUs = 0.018f, kWideSplitUs = 2.5f;
-
-static float wide_cost(int64_t dp_rounds, int64_t R, int c, int nkb, int P, int C) {
-    const int64_t n = R * c;
-    const int w = (nkb + c - 1) / c;
-    const int64_t full = n / P, rem = n % P;
-    float us = (float)dp_rounds * nkb * kWideRoundUs + (float)full * w * kWideRoundUs;
-    if (rem) us += (float)w * (rem > C ? kWidePairUs + kWidePairSlopeUs * (float)(rem - C) / (float)C : kWideLoneUs);
-    if (c > 1) us += kWideSplitUs + kWideSlotUs * (float)n;
-    return us;
-}
-
-/* (whole tiles, pieces) of T tiles of K; wide: the 128 x 128 tile's model,
- * else the 64 x 256 one's. */
-static void tail_plan(bool wide, int T, int nkb, int cus, size_t slot_floats, size_t max_slot_floats, int *dp_tiles,
-                      int *pieces) {
+/* Whole-tile workgroups and K pieces of T tiles on `cus` compute units, the
+ * least modelled time. The device keeps 2 workgroups per CU resident, so P =
+ * 2 * cus run per round. The whole tiles are a multiple of P (all full
+ * rounds, or one round fewer); the R tiles left are cut into c K ranges (c =
+ * 1: whole as well). The split tiles' slots must fit max_slot_floats. */
+static void tail_plan(const sera_tile_cost &k, int T, int nkb, int cus, size_t slot_floats, size_t max_slot_floats,
+                      int *dp_tiles, int *pieces) {
     const int C = cus > 0 ? cus : kModelCUs;
     const int P = 2 * C;
     const int rounds = T / P;
-    auto cost = [&](int64_t dp_rounds, int64_t R, int c) {
-        return wide ? wide_cost(dp_rounds, R, c, nkb, P, C) : tail_cost(dp_rounds, R, c, nkb, P, C);
-    };
     int best_dp = T, best_c = 1;
-    float best = cost(rounds, T - (int64_t)rounds * P, 1);
+    float best = sera_plan_cost(&k, rounds, T - (long)rounds * P, 1, nkb, C);
     for (int fold = 0; fold <= (rounds > 0 ? 1 : 0); fold++) {
         const int dp = (rounds - fold) * P;
         const int R = T - dp;
         if (R == 0) continue;
         for (int c = 2; c <= (nkb < 16 ? nkb : 16); c++) {
             if ((size_t)R * c * slot_floats > max_slot_floats) break;
-            const float us = cost(rounds - fold, R, c);
+            const float us = sera_plan_cost(&k, rounds - fold, R, c, nkb, C);
             if (us < best) { best = us; best_dp = dp; best_c = c; }
         }
     }
@@ -1550,14 +1524,14 @@ static void tail_plan(bool wide, int T, int nkb, int cus, size_t slot_floats, si
 
 extern "C" void sera_mmq_tail_plan(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles,
                                    int *pieces) {
-    tail_plan(mmq_wide(M, N), sera_mmq_tiles(M, N), K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles,
+    tail_plan(tile_cost(M, N), sera_mmq_tiles(M, N), K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles,
               pieces);
 }
 
 /* The same for the `tiles` wide tiles of a group (sera_mmq_group_tiles). */
 extern "C" void sera_mmq_group_plan(int tiles, int M, int K, int cus, size_t max_slot_floats, int *dp_tiles,
                                     int *pieces) {
-    tail_plan(true, tiles, K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles, pieces);
+    tail_plan(kCostWide, tiles, K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles, pieces);
 }
 
 /* Floats of the tail schedule's slots and ints of its counters. */

@@ -17,6 +17,27 @@
 extern "C" {
 #endif
 
+/* What a tile kernel costs under the tail schedule, us (fitted constants
+ * beside each tile). With C compute units, P = 2 * C workgroups to a round: a
+ * full round of workgroups of w super-blocks w * step + fix; a last round
+ * that leaves every CU at most one workgroup w * lone + lone_fix (after
+ * whole-tile rounds w * lone + after: it starts while they end), above that w
+ * * (from pair just past one per CU to step at P) + fix; and n workgroups
+ * that share tiles in c pieces split + n * slot (a tile's sums written
+ * through and read back each) + c * piece (the last piece reads the others).
+ * The product: dp_rounds rounds of whole tiles, then R tiles in c pieces (c =
+ * 1: whole as well). */
+typedef struct { float step, fix, lone, lone_fix, pair, slot, split, piece, after; } sera_tile_cost;
+static inline float sera_plan_cost(const sera_tile_cost *k, long dp_rounds, long R, int c, int nkb, int C) {
+    const long P = 2l * C, n = R * c, full = n / P, rem = n % P;
+    const float w = (float)((nkb + c - 1) / c);
+    float us = (float)dp_rounds * ((float)nkb * k->step + k->fix) + (float)full * (w * k->step + k->fix);
+    if (rem > C) us += w * (k->pair + (k->step - k->pair) * (float)(rem - C) / (float)C) + k->fix;
+    else if (rem) us += w * k->lone + (dp_rounds ? k->after : k->lone_fix);
+    if (c > 1) us += k->split + k->slot * (float)n + k->piece * (float)c;
+    return us;
+}
+
 /* ---- q8_quantize.hip: activation stages ------------------------------- */
 hipError_t sera_launch_q8_1_row(const float *x, int M, int K, void *stage, hipStream_t stream);
 hipError_t sera_launch_q8_1_mmq(const float *x, int M, int Mpad, int K, void *stage, hipStream_t stream);

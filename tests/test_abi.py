@@ -306,6 +306,19 @@ def test_mmq_split_rule_picks_measured_best():
                     assert K // 256 // s >= 2 and L.sera_q4k_mmq_tiles(M, N) * s <= 2048, (M, N, K, s)
 
 
+def test_tail_plan_keeps_short_products_whole(L):
+    """Products whose M * N is no multiple of 4 run under the tail schedule:
+    on 16- and 32-token and 64 x 128 tiles a short K is not worth its pieces
+    (a call at 11 tokens of 15767 x 768 whole 10.7 us, in pieces 11.9, at 26 of
+    26351 x 512 10.7 and 12.2), a long one is."""
+    dp, pieces = ctypes.c_int(), ctypes.c_int()
+    for M, N, K, whole in ((11, 15767, 768, True), (26, 26351, 512, True), (56, 13165, 512, True), (203, 1333, 1792, False),
+                           (19, 3001, 2048, False), (13, 1001, 2304, False), (65, 511, 5120, False)):
+        L.sera_mmq_tail_plan(M, N, K, 256, ctypes.c_size_t(1 << 28), ctypes.byref(dp), ctypes.byref(pieces))
+        tiles = L.sera_q4k_mmq_tiles(M, N)
+        assert ((dp.value, pieces.value) == (tiles, 1)) == whole, (M, N, K, dp.value, pieces.value)
+
+
 def test_kernel_launch_counts(L):
     """quantize + matmul (+ the split-K reduce when an MMQ launch splits K)."""
     assert L.sera_q4k_kernel_launches(1, 25600, 5120) == 2          # dot4 MMVQ
