@@ -739,6 +739,24 @@ extern "C" int sera_q6k_mmvq(uint32_t qtype, const void *W, const void *row_stag
 }
 
 namespace {
+/* Pieces of T Q6_K tiles whose M * N is no multiple of 4 (split-K's 16-byte
+ * reduce cannot serve them): the least modelled time of 1 (whole) to
+ * max_pieces, one round of workgroups. Fitted on MI355X to the kernel's times
+ * under every piece count of 190 random shapes with the 32-token tile and 33
+ * with the 64-token one, both layouts: 2.1% and 3.1% over the fastest, which
+ * may need more than one round. As many pieces of two super-blocks as a round
+ * holds cost 4% more, and on a short K more than whole tiles (22365 x 1280 at
+ * 13 tokens 14.8 us a call whole, 16.8 in pieces). */
+int q6k_odd_pieces(int T, int tile_tokens, int nkb, int max_pieces) {
+    static constexpr sera_tile_cost k32 = {2.32f, 1.42f, 2.32f, 2.41f, 3.58f, 0.013f, 1.0f, 0.38f, 2.41f};
+    static constexpr sera_tile_cost k64 = {4.33f, 3.61f, 3.52f, 2.23f, 4.9f, 0.015f, 1.47f, 0.42f, 2.23f};
+    const sera_tile_cost *k = tile_tokens == 64 ? &k64 : &k32;
+    int best = 1;
+    for (int c = 2; c <= max_pieces; c++)
+        if (sera_plan_cost(k, 0, T, c, nkb, g_cus) < sera_plan_cost(k, 0, T, best, nkb, g_cus)) best = c;
+    return best;
+}
+
 /* Q6_K tile kernel schedule: the tail (every tile cut into K pieces handed
  * off through counters, no reduce launch) when one round of resident
  * workgroups (P = 2 per CU) gives each tile at least 4 pieces of at least 5
@@ -751,17 +769,15 @@ namespace {
 bool q6k_tail_plan(int M, int N, int K, size_t cap, int *dp, int *pieces) {
     if (!g_counters || g_cus <= 0) return false;
     const int T = sera_q6k_mmq_tiles(M, N, K);
-    int p = 2 * g_cus / T;
-    const int nkb = K / Q4K_QK;
+    const int p = 2 * g_cus / T, nkb = K / Q4K_QK;
+    if (T > kFewtokCounterBase) return false;
+    int pc = p < 63 ? p : 63;
     if (((size_t)M * N) % 4 != 0) {
-        /* split-K's 16-byte reduce cannot serve these: pieces of at least
-         * two super-blocks, else whole tiles */
-        if (p > nkb / 2) p = nkb / 2;
-        if (T > kFewtokCounterBase || p < 2) return false;
-    } else if (T > kFewtokCounterBase || p < 4 || nkb < 5 * p) {
+        pc = q6k_odd_pieces(T, sera_q6k_mmq_tile_tokens(M, N, K), nkb, pc < nkb ? pc : nkb);
+        if (pc < 2) return false;
+    } else if (p < 4 || nkb < 5 * p) {
         return false;
     }
-    const int pc = p < 63 ? p : 63;
     if (sera_q6k_mmq_tail_slot_floats(M, N, K, 0, pc) > cap) return false;
     *dp = 0;
     *pieces = pc;

@@ -166,6 +166,16 @@ def test_rmsnorm_q6k_stage_pieces(torch, M, K):  # noqa: F811
     assert np.array_equal(d[:, rows].T, np.asarray(xd).reshape(len(rows), K // 32))
 
 
+def test_q6k_odd_products_plan(torch):  # noqa: F811
+    """Odd Q6_K products are cut along K only where that is modelled (and was
+    measured) faster than whole tiles."""
+    q3q4.Linear(device=0, max_tokens=512, max_features=32768, max_k=25600)
+    for M, N, K, whole in ((13, 22365, 1280, True), (39, 10343, 1280, True), (11, 1241, 2048, False), (31, 313, 25600, False),
+                           (203, 1131, 2048, False), (443, 4369, 1536, True)):
+        plan = q3q4.q6k_mmq_tail_plan(M, N, K)
+        assert (plan is None) == whole, (M, N, K, plan)
+
+
 # |x| above 8.3e6 overflows the fp16 token scale: the formula's (I * sw) * inf is +-inf, and NaN only where the dot or the
 # scale is zero or infinities of both signs meet. M = 193: both token-tile bodies; the last token's second block overflows too.
 @pytest.mark.parametrize("dp,pieces", [(10 ** 6, 1), (0, 2)])
