@@ -183,14 +183,21 @@ int sera_q4k_mmq_splits(int M, int N, int K);
 int sera_q4k_mmq_streamk(const void *W, const void *mmq_stage, float *Y, float *slots, int *counters,
                          int M, int N, int K, int wgs, void *stream);
 int sera_q4k_mmq_streamk_wgs(int M);   /* resident workgroups for M tokens (after init) */
-/* Schedule of the MMQ tile kernels for this shape (after init): 2 = whole
- * tiles + split tail (M > 32, and where M*N is no multiple of 4; below), 1 = stream-K
- * (16- and 32-token tiles, M <= 32, from one full round of resident
- * workgroups of tiles), 0 = plain tiles / split-K with the split count of
- * sera_q4k_mmq_splits (a per-CU cost model fitted to MI355X timings); -1
- * for a bad shape. sera_q4k_dense runs it where sera_q4k_mmq_uses_fewtok
- * is 0. */
+/* Schedule of the MMQ tile kernels for this shape (after init). With P =
+ * twice the CU count and T = sera_q4k_mmq_tiles(M, N):
+ *   2 = whole tiles + split tail (below): for M > 32 where T > P/8; and where
+ *       M*N is no multiple of 4, for M > 32 always, else where T < P;
+ *   1 = stream-K (M <= 32 and P <= T < 4P);
+ *   0 = plain tiles / split-K with the split count of sera_q4k_mmq_splits (a
+ *       per-CU cost model fitted to MI355X timings);
+ *   -1 for a bad shape.
+ * sera_q4k_dense runs it where sera_q4k_mmq_uses_fewtok is 0. Where T counts
+ * 128 x 128 tiles but 64 x 256 ones are modelled faster (padding to 128
+ * tokens, short K: sera_q4k_mmq_on_64x256 is 1, after init and with an arena),
+ * it runs schedule 2 on those, with a plan of its own; the explicit entry
+ * points always run the tiles of sera_q4k_mmq_tiles. */
 int sera_q4k_mmq_schedule(int M, int N, int K);
+int sera_q4k_mmq_on_64x256(int M, int N, int K);
 
 /* MMQ kernel under the tail schedule (the role of mul_mat_q's stream-K
  * decomposition, cuda/mmq/mmq.cuh:3641-4352, for the last round of tiles
@@ -205,7 +212,7 @@ int sera_q4k_mmq_schedule(int M, int N, int K);
  * the product to Y. sera_q4k_mmq_tail_plan gives the schedule's own choice
  * (after init; slots limited to max_slot_floats, or with 0 to what the
  * attached arena holds after the stage: the plan sera_q4k_dense runs where
- * sera_q4k_mmq_schedule is 2). */
+ * sera_q4k_mmq_schedule is 2 and sera_q4k_mmq_on_64x256 is 0). */
 int sera_q4k_mmq_tail_qt(uint32_t qtype, const void *W, const void *mmq_stage, float *Y, float *slots, int *counters,
                          int M, int N, int K, int dp_tiles, int pieces, int accum, void *stream);
 int sera_q4k_mmq_tail_plan(int M, int N, int K, size_t max_slot_floats, int *dp_tiles, int *pieces);
@@ -216,9 +223,9 @@ size_t sera_q4k_mmq_tail_slot_floats(int M, int N, int dp_tiles, int pieces);
  * up, down, the LM head); 0 otherwise. No counterpart in the reference
  * (mul_mat_q has one kernel family); a dispatch query. */
 int sera_q4k_mmq_uses_fewtok(int M, int N, int K);
-/* MMQ output tiles for M tokens of N rows: 16, 32 or 64 tokens by 256 rows,
- * or 64 by 128 where 256-row tiles would number at most 64, else 128 by 128
- * from 65 tokens on. */
+/* MMQ output tiles for M tokens of N rows: 16 (M <= 16), 32 (M <= 32) or 64
+ * tokens by 256 rows; 64 by 128 where M > 32 and the 64 by 256 ones would
+ * number at most 64; else 128 by 128 where M > 64 and N is a multiple of 4. */
 int sera_q4k_mmq_tiles(int M, int N);
 /* Floats of one stream-K or tail slot for M tokens (the largest tile's). */
 int sera_q4k_mmq_slot_floats(int M);

@@ -1482,13 +1482,14 @@ extern "C" hipError_t sera_launch_q4k_mmq_streamk_acc(uint32_t qtype, const void
  *     256 tile's constants cost these three 3-5%, at most 37%, above all by
  *     splitting a short K that runs faster whole (15767 x 768 at 11 tokens:
  *     62 whole tiles 10.7 us a call, in 3 pieces 11.9);
- *   64 x 256 tile: 14 Qwen3-32B shapes (q, k/v, o, gate/up, down at 64-2048
- *     tokens), at most 1.6%;
- *   128 x 128 tile: 13 shapes of 100-2048 tokens, at most 4%. */
+ *   64 x 256 tile, 948 shapes of 33-2048 tokens: 0.5%, at most 13% (without a
+ *     cost per round 9% and 2.7 times: 770 tiles of 4 super-blocks 49 us
+ *     whole, 130 in pieces);
+ *   128 x 128 tile, 828 shapes of 65-2048 tokens: 0.5%, at most 11%. */
 static constexpr sera_tile_cost kCost16 = {3.1f, 0.0f, 2.17f, 2.25f, 2.9f, 0.021f, 1.35f, 0.37f, 2.25f};
 static constexpr sera_tile_cost kCost8192 = {2.9f, 1.7f, 2.55f, 3.05f, 3.5f, 0.018f, 1.0f, 0.44f, 3.05f};
-static constexpr sera_tile_cost kCost64x256 = {5.0f, 0.0f, 3.2f, 0.0f, 5.0f, 0.0f, 0.0f, 1.5f, 0.0f};
-static constexpr sera_tile_cost kCostWide = {5.4f, 0.0f, 3.25f, 0.0f, 4.5f, 0.018f, 2.5f, 0.0f, 0.0f};
+static constexpr sera_tile_cost kCost64x256 = {4.52f, 7.27f, 3.16f, 6.24f, 4.64f, 0.009f, 5.17f, 0.46f, 2.51f};
+static constexpr sera_tile_cost kCostWide = {4.26f, 9.21f, 2.89f, 6.04f, 4.0f, 0.003f, 3.96f, 0.68f, 2.48f};
 
 static const sera_tile_cost &tile_cost(int M, int N) {
     if (mmq_wide(M, N)) return kCostWide;
@@ -1497,12 +1498,12 @@ static const sera_tile_cost &tile_cost(int M, int N) {
 }
 
 /* Whole-tile workgroups and K pieces of T tiles on `cus` compute units, the
- * least modelled time. The device keeps 2 workgroups per CU resident, so P =
+ * least modelled time, which it returns. The device keeps 2 workgroups per CU resident, so P =
  * 2 * cus run per round. The whole tiles are a multiple of P (all full
  * rounds, or one round fewer); the R tiles left are cut into c K ranges (c =
  * 1: whole as well). The split tiles' slots must fit max_slot_floats. */
-static void tail_plan(const sera_tile_cost &k, int T, int nkb, int cus, size_t slot_floats, size_t max_slot_floats,
-                      int *dp_tiles, int *pieces) {
+static float tail_plan(const sera_tile_cost &k, int T, int nkb, int cus, size_t slot_floats, size_t max_slot_floats,
+                       int *dp_tiles, int *pieces) {
     const int C = cus > 0 ? cus : kModelCUs;
     const int P = 2 * C;
     const int rounds = T / P;
@@ -1520,12 +1521,32 @@ static void tail_plan(const sera_tile_cost &k, int T, int nkb, int cus, size_t s
     }
     *dp_tiles = best_dp;
     *pieces = best_c;
+    return best;
 }
 
 extern "C" void sera_mmq_tail_plan(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles,
                                    int *pieces) {
     tail_plan(tile_cost(M, N), sera_mmq_tiles(M, N), K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles,
               pieces);
+}
+
+/* 64 x 256 tiles in place of the 128 x 128 ones of sera_mmq_tiles: their
+ * number and plan where they are modelled faster (by 1%, the models' ties being
+ * the wide tile's), else 0. That is where the padding to 128 tokens adds a
+ * round or much of one, and on a K of one or two super-blocks, whose prologue
+ * and stores the wide tile hides less. us a call, 64 x 256 / wide: 565 x 6704
+ * (243 / 265 tiles) x 256 12.7 / 14.6, x 1024 23.6 / 27.8; 541 x 14284 x 768
+ * 26.8 / 34.3, 386 x 5644 x 8192 73.7 / 87.5; the other way 412 x 9848 x 768
+ * 38.5 / 24.0, 2048 x 4096 x 2048 57.7 / 56.4. Over 828 random shapes the
+ * choice costs 0.6% over the faster tile under its fastest plan, at most 11%;
+ * always the wide one under its earlier plan 2.2%, up to 38%. */
+extern "C" int sera_mmq_plan64(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles, int *pieces) {
+    if (!mmq_wide(M, N)) return 0;
+    int dp, pc;
+    const size_t slot = sera_mmq_slot_floats(M);
+    const int T = ((M + 63) / 64) * ((N + 255) / 256);
+    const float wide = tail_plan(kCostWide, sera_mmq_tiles(M, N), K / Q4K_QK, cus, slot, max_slot_floats, &dp, &pc);
+    return tail_plan(kCost64x256, T, K / Q4K_QK, cus, slot, max_slot_floats, dp_tiles, pieces) < 0.99f * wide ? T : 0;
 }
 
 /* The same for the `tiles` wide tiles of a group (sera_mmq_group_tiles). */
@@ -1544,7 +1565,8 @@ template <int TT, int WGT, int WGN, int WPE, int PR = 0>
 static hipError_t launch_mmq_tail_cfg(int tiled, const uint8_t *W, const int8_t *xq, const uint32_t *xds, float *y,
                                       float *slots, int *counters, int M, int N, int K, int dp_tiles, int pieces,
                                       int accum, hipStream_t s) {
-    const int T = sera_mmq_tiles(M, N);
+    constexpr int BM = MmqShape<TT, WGT, WGN, PR>::BM, BN = MmqShape<TT, WGT, WGN, PR>::BN;
+    const int T = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     const int grid = dp_tiles + (T - dp_tiles) * pieces;
     hipLaunchKernelGGL((sera_q4k_mmq_tail_kernel<TT, WGT, WGN, WPE, PR>), dim3(grid), dim3(256), 0, s, W, xq, xds, y,
                        slots, counters, M, N, K, dp_tiles, pieces, accum, tiled);
@@ -1628,4 +1650,22 @@ extern "C" hipError_t sera_launch_q4k_mmq_tail_acc(uint32_t qtype, const void *W
                                                 accum, s);
     return launch_mmq_tail_cfg<2, 1, 4, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, dp_tiles, pieces, accum,
                                             s);
+}
+
+/* The tail schedule on 64 x 256 tiles with the plan of sera_mmq_plan64: slots
+ * (tiles - dp_tiles) * pieces * sera_mmq_slot_floats(M) floats, counters as
+ * above. */
+extern "C" hipError_t sera_launch_q4k_mmq_tail64_acc(uint32_t qtype, const void *W, const void *stage, float *y,
+                                                     float *slots, int *counters, int M, int N, int K, int dp_tiles,
+                                                     int pieces, int accum, hipStream_t s) {
+    const int tiled = qtype == SERA_QTYPE_Q4K_TILED;
+    const int T = ((M + 63) / 64) * ((N + 255) / 256);
+    if ((!tiled && qtype != 12u) || (tiled && N % Q4K_TILE_ROWS) || M <= 64 || dp_tiles < 0 || dp_tiles > T ||
+        pieces < 1 || pieces > K / Q4K_QK)
+        return hipErrorInvalidValue;
+    const sera_stage_layout L = sera_mmq_stage_layout((size_t)sera_mmq_padded_rows(M), (size_t)K);
+    const char *base = (const char *)stage;
+    return launch_mmq_tail_cfg<2, 1, 4, 2>(tiled, (const uint8_t *)W, (const int8_t *)(base + L.qs),
+                                           (const uint32_t *)(base + L.ds), y, slots, counters, M, N, K, dp_tiles,
+                                           pieces, accum, s);
 }

@@ -81,6 +81,10 @@ hipError_t sera_launch_q4k_mmq_streamk_acc(uint32_t qtype, const void *W, const 
                                            int *counters, int M, int N, int K, int P, int accum, hipStream_t s);
 void sera_mmq_tail_plan(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles, int *pieces);
 size_t sera_mmq_tail_slot_floats(int M, int N, int dp_tiles, int pieces);
+int sera_mmq_plan64(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles, int *pieces);
+hipError_t sera_launch_q4k_mmq_tail64_acc(uint32_t qtype, const void *W, const void *stage, float *y, float *slots,
+                                          int *counters, int M, int N, int K, int dp_tiles, int pieces, int accum,
+                                          hipStream_t s);
 int sera_mmq_group_tiles(int M, int count, const int *N);
 void sera_mmq_group_plan(int tiles, int M, int K, int cus, size_t max_slot_floats, int *dp_tiles, int *pieces);
 hipError_t sera_launch_q4k_mmq_wide_group(uint32_t qtype, int count, const void *const *W, float *const *y,

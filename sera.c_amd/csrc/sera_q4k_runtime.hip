@@ -433,7 +433,7 @@ bool tail_rule(int M, int N) {
 }
 
 struct MmqPlan {
-    int kind;        /* 0 split-K (splits), 1 stream-K, 2 tail (dp_tiles, pieces) */
+    int kind;        /* 0 split-K (splits), 1 stream-K, 2 tail (dp_tiles, pieces), 3 tail on 64 x 256 tiles */
     int splits, dp_tiles, pieces;
     size_t partial_floats;
 };
@@ -442,6 +442,12 @@ struct MmqPlan {
 MmqPlan mmq_plan(int M, int N, int K, size_t cap, bool have_counters) {
     MmqPlan p = {0, 1, 0, 1, 0};
     if (have_counters && tail_rule(M, N)) {
+        const int t64 = sera_mmq_plan64(M, N, K, g_cus, cap, &p.dp_tiles, &p.pieces);
+        if (t64 > 0 && (p.pieces == 1 || t64 - p.dp_tiles <= kFewtokCounterBase)) {
+            p.kind = 3;
+            p.partial_floats = p.pieces > 1 ? (size_t)(t64 - p.dp_tiles) * p.pieces * sera_mmq_slot_floats(M) : 0;
+            return p;
+        }
         sera_mmq_tail_plan(M, N, K, g_cus, cap, &p.dp_tiles, &p.pieces);
         const int R = sera_mmq_tiles(M, N) - p.dp_tiles;
         if (p.pieces == 1 || R <= kFewtokCounterBase) {
@@ -465,6 +471,9 @@ MmqPlan mmq_plan(int M, int N, int K, size_t cap, bool have_counters) {
 
 hipError_t mmq_launch(const MmqPlan &p, uint32_t qt, const void *W, const void *stage, float *Y, float *partial,
                       int M, int N, int K, int accum, hipStream_t s) {
+    if (p.kind == 3)
+        return sera_launch_q4k_mmq_tail64_acc(qt, W, stage, Y, partial, g_counters, M, N, K, p.dp_tiles, p.pieces,
+                                              accum, s);
     if (p.kind == 2)
         return sera_launch_q4k_mmq_tail_acc(qt, W, stage, Y, partial, g_counters, M, N, K, p.dp_tiles, p.pieces,
                                             accum, s);
@@ -572,21 +581,30 @@ extern "C" int sera_q4k_dense_qt(uint32_t qtype, const void *W, const float *X, 
 
 extern "C" int sera_q4k_mmq_streamk_wgs(int M) { return M > 0 ? streamk_wgs(M) : 0; }
 
+namespace {
+/* scratch floats the attached arena holds after the stage of M tokens of K */
+size_t arena_slot_floats(int M, int K) {
+    const size_t stage = sera_mmq_stage_layout((size_t)sera_mmq_padded_rows(M), (size_t)K).total;
+    return g_arena && g_arena_bytes > stage ? (g_arena_bytes - stage) / sizeof(float) : 0;
+}
+}  // namespace
+
 extern "C" int sera_q4k_mmq_schedule(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % Q4K_QK) return -1;
     if (tail_rule(M, N)) return 2;
     return streamk_rule(M, N, K) ? 1 : 0;
 }
 
+extern "C" int sera_q4k_mmq_on_64x256(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % Q4K_QK) return 0;
+    return mmq_plan(M, N, K, arena_slot_floats(M, K), g_counters != nullptr).kind == 3;
+}
+
 extern "C" int sera_q4k_mmq_tail_plan(int M, int N, int K, size_t max_slot_floats, int *dp_tiles, int *pieces) {
     if (M <= 0 || N <= 0 || K <= 0 || K % Q4K_QK || !dp_tiles || !pieces)
         return fail(-1, "sera_q4k_mmq_tail_plan: bad arguments");
     if (g_cus <= 0) return fail(-1, "sera_q4k_mmq_tail_plan: not initialised (the CU count is unknown)");
-    if (max_slot_floats == 0) {
-        /* what sera_q4k_dense would use: the attached arena after the stage */
-        const size_t stage = sera_mmq_stage_layout((size_t)sera_mmq_padded_rows(M), (size_t)K).total;
-        max_slot_floats = g_arena && g_arena_bytes > stage ? (g_arena_bytes - stage) / sizeof(float) : 0;
-    }
+    if (max_slot_floats == 0) max_slot_floats = arena_slot_floats(M, K);   /* what sera_q4k_dense would use */
     sera_mmq_tail_plan(M, N, K, g_cus, max_slot_floats, dp_tiles, pieces);
     return 0;
 }

@@ -120,6 +120,7 @@ def load():
         "sera_q4k_mmq_streamk": ([P, P, P, P, P, I, I, I, I, P], I),
         "sera_q4k_mmq_streamk_wgs": ([I], I),
         "sera_q4k_mmq_schedule": ([I, I, I], I),
+        "sera_q4k_mmq_on_64x256": ([I, I, I], I),
         "sera_q4k_mmq_tail_qt": ([U32, P, P, P, P, P, I, I, I, I, I, I, P], I),
         "sera_q4k_mmq_tail_plan": ([I, I, I, SZ, ctypes.POINTER(I), ctypes.POINTER(I)], I),
         "sera_q4k_mmq_tail_slot_floats": ([I, I, I, I], SZ),

@@ -319,6 +319,26 @@ def test_tail_plan_keeps_short_products_whole(L):
         assert ((dp.value, pieces.value) == (tiles, 1)) == whole, (M, N, K, dp.value, pieces.value)
 
 
+def test_prefill_tile_by_modelled_time(L):
+    """128 x 128 or 64 x 256 tiles, whichever was measured (and is modelled)
+    faster: the wide tile on the Qwen3-32B shapes and most others, not where
+    its padding to 128 tokens adds a round or K is a super-block or two."""
+    dp, pieces = ctypes.c_int(), ctypes.c_int()
+
+    def tiles64(M, N, K, cap=1 << 30):
+        return L.sera_mmq_plan64(M, N, K, 256, ctypes.c_size_t(cap), ctypes.byref(dp), ctypes.byref(pieces))
+
+    for M, N, K in ((512, 25600, 5120), (2048, 25600, 5120), (512, 5120, 25600), (512, 8192, 5120), (256, 5120, 8192),
+                    (412, 9848, 768), (2048, 4096, 2048), (64, 25600, 5120), (565, 6702, 1024), (512, 1024, 5120)):
+        assert tiles64(M, N, K) == 0, (M, N, K)
+    for M, N, K in ((565, 6704, 256), (565, 6704, 512), (565, 6704, 1024), (190, 20900, 256), (190, 20900, 1024),
+                    (541, 14284, 768), (386, 5644, 8192), (2048, 4096, 256)):
+        assert tiles64(M, N, K) == -(-M // 64) * -(-N // 256), (M, N, K)
+        assert 0 <= dp.value <= tiles64(M, N, K) and 1 <= pieces.value <= K // 256
+    assert tiles64(386, 5644, 8192) and (dp.value, pieces.value) == (0, 3)
+    assert tiles64(386, 5644, 8192, cap=161 * 2 * 64 * 256) == 0 or pieces.value <= 2     # slots for two pieces
+
+
 def test_kernel_launch_counts(L):
     """quantize + matmul (+ the split-K reduce when an MMQ launch splits K)."""
     assert L.sera_q4k_kernel_launches(1, 25600, 5120) == 2          # dot4 MMVQ

@@ -166,6 +166,32 @@ def test_rmsnorm_q6k_stage_pieces(torch, M, K):  # noqa: F811
     assert np.array_equal(d[:, rows].T, np.asarray(xd).reshape(len(rows), K // 32))
 
 
+# 64 x 256 tiles in place of the wide ones: whole tiles and all in three pieces, both layouts, plain and
+# accumulating, through the boundary and as a group of one
+@pytest.mark.parametrize("M,N,K", [(131, 16532, 256), (129, 5392, 2304)])
+def test_narrow_tile_where_it_is_faster(torch, M, N, K):  # noqa: F811
+    L = q3q4.load()
+    lin = q3q4.Linear(device=0, max_tokens=192, max_features=16640, max_k=2304)
+    assert L.sera_q4k_mmq_schedule(M, N, K) == 2 and L.sera_q4k_mmq_on_64x256(M, N, K) == 1
+    rng = np.random.default_rng(M + N + K)
+    W, X = exact_inputs(rng, M, N, K)
+    ref = expected(W, X, N, K)
+    base = rng.integers(-4, 5, (M, N)).astype(np.float32)
+    layouts = [(12, W)] + ([(q3q4.QTYPE_Q4K_TILED, q3q4.q4k_tiled_bytes(W, N, K))] if N % 16 == 0 else [])
+    for qt, w in layouts:
+        Wd, Xd, g = dev(torch, w), dev(torch, X), q3q4.bind_geometry(qt, K, N)
+        say(f"case 64 x 256 tail qt={qt} M={M} N={N} K={K}")
+        y = nan_out(torch, M, N)
+        lin(g, Wd, Xd, y)
+        torch.cuda.synchronize()
+        assert_bits(y, ref, "boundary")
+        y.copy_(torch.from_numpy(base))
+        q3q4.linear_group([g], [Wd], [y], Xd, flags=q3q4.LIN_ACCUMULATE)
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy(), base + ref.astype(np.float32))
+    assert int(lin.workspace[:256 << 10].to(torch.int32).abs().sum()) == 0, "tile counters not reset"
+
+
 def test_q6k_odd_products_plan(torch):  # noqa: F811
     """Odd Q6_K products are cut along K only where that is modelled (and was
     measured) faster than whole tiles."""
