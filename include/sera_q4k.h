@@ -430,8 +430,13 @@ int sera_weight_upload(uint32_t qtype, int N, int K, const void *host_gguf, void
  * the activations are quantized once for the group (q/k/v and gate/up read
  * the same normed input). At decode (Q4_K, M <= 8) the matrices the dot4
  * MMVQ kernel takes (sera_q4k_vec_uses_fewtok == 0) share one grouped
- * launch and the others run the few-token kernel one by one; a Q6_K group
- * shares one stage, so its largest matrix picks the kernel
+ * launch and the others run the few-token kernel one by one. Over 64 tokens
+ * a Q4_K group (every N a multiple of 4) runs as one launch of 128 x 128
+ * tiles where that is modelled faster, its K ranges planned over all its
+ * tiles: a product's fp32 sums may then be split elsewhere than those of the
+ * separate call (the same terms, added in another order; repeats are bit for
+ * bit). Outputs that share memory run one by one, in the order given. A Q6_K
+ * group shares one stage, so its largest matrix picks the kernel
  * (sera_q6k_vec_uses_tile_qt). Arithmetic per product as q3_cuda_q4k_linear (MMVQ
  * formula for M <= 8, MMQ above). gamma and X2 must be 16-byte aligned.
  * Uses the arena of sera_q4k_set_arena / q3_cuda_q4k_linear_set_workspace;

@@ -1561,12 +1561,6 @@ extern "C" int sera_mmq_plan64(int M, int N, int K, int cus, size_t max_slot_flo
     return tail_plan(kCost64x256, T, K / Q4K_QK, cus, slot, max_slot_floats, dp_tiles, pieces) < 0.99f * wide ? T : 0;
 }
 
-/* The same for the `tiles` wide tiles of a group (sera_mmq_group_tiles). */
-extern "C" void sera_mmq_group_plan(int tiles, int M, int K, int cus, size_t max_slot_floats, int *dp_tiles,
-                                    int *pieces) {
-    tail_plan(kCostWide, tiles, K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats, dp_tiles, pieces);
-}
-
 /* Floats of the tail schedule's slots and ints of its counters. */
 extern "C" size_t sera_mmq_tail_slot_floats(int M, int N, int dp_tiles, int pieces) {
     const int R = sera_mmq_tiles(M, N) - dp_tiles;
@@ -1585,21 +1579,42 @@ static hipError_t launch_mmq_tail_cfg(int tiled, const uint8_t *W, const int8_t 
     return hipGetLastError();
 }
 
-/* Wide tiles of a group of matrices (M > 64), or 0 where the group is better
- * run matrix by matrix: one matrix, a row count that is no multiple of 4, or
- * no more than kNarrowTileMax 64 x 256 tiles in all. One launch for the group
- * against one per matrix (k and v on their own narrow tiles): the linear steps
- * of a Qwen3-32B layer at 512 tokens 795 -> 739 us on MI355X, with the plan
- * below. */
-extern "C" int sera_mmq_group_tiles(int M, int count, const int *N) {
+/* Modelled us of one product's kernel as a call of its own. */
+static float product_us(int M, int N, int nkb, int cus, size_t max_slot_floats) {
+    int dp, pieces;
+    const size_t slot = sera_mmq_slot_floats(M);
+    const float us = tail_plan(tile_cost(M, N), sera_mmq_tiles(M, N), nkb, cus, slot, max_slot_floats, &dp, &pieces);
+    if (!mmq_wide(M, N)) return us;
+    const int T = ((M + 63) / 64) * ((N + 255) / 256);
+    const float us64 = tail_plan(kCost64x256, T, nkb, cus, slot, max_slot_floats, &dp, &pieces);
+    return us64 < us ? us64 : us;
+}
+
+/* Wide tiles of a group of matrices (M > 64) as one launch, and their plan, or
+ * 0 where the group runs matrix by matrix: one matrix, a row count that is no
+ * multiple of 4, no more than kNarrowTileMax 64 x 256 tiles in all, or a
+ * modelled time above the separate products' with kLaunchUs for each launch
+ * saved. One launch against one per matrix, on MI355X: the linear steps of a
+ * Qwen3-32B layer at 512 tokens 795 -> 739 us, 411 random groups of 65-2048
+ * tokens 0.63 of the time; the other way where the padding to 128 tokens costs
+ * more than the launches, us in one launch / in two: 2 x 42624 x 512 at 140
+ * tokens 47.4 / 39.9, x 2048 at 135 tokens 120.6 / 99.2. */
+static constexpr float kLaunchUs = 4.0f;
+extern "C" int sera_mmq_group_plan(int M, int count, const int *N, int K, int cus, size_t max_slot_floats,
+                                   int *dp_tiles, int *pieces) {
     if (M <= 64 || count < 2 || count > 4) return 0;
     int64_t narrow = 0, wide = 0;
+    float alone = kLaunchUs * (float)(count - 1);
     for (int i = 0; i < count; i++) {
         if (N[i] % 4) return 0;
         narrow += (int64_t)((M + 63) / 64) * ((N[i] + 255) / 256);
         wide += (int64_t)((M + kWideBM - 1) / kWideBM) * ((N[i] + kWideBN - 1) / kWideBN);
+        alone += product_us(M, N[i], K / Q4K_QK, cus, max_slot_floats);
     }
-    return narrow > kNarrowTileMax && wide <= 0x7fffffff ? (int)wide : 0;
+    if (narrow <= kNarrowTileMax || wide > 0x7fffffff) return 0;
+    const float us = tail_plan(kCostWide, (int)wide, K / Q4K_QK, cus, sera_mmq_slot_floats(M), max_slot_floats,
+                               dp_tiles, pieces);
+    return us <= alone ? (int)wide : 0;
 }
 
 /* Wide tiles of up to four N[i] x K matrices on one stage, under the tail

@@ -85,8 +85,8 @@ int sera_mmq_plan64(int M, int N, int K, int cus, size_t max_slot_floats, int *d
 hipError_t sera_launch_q4k_mmq_tail64_acc(uint32_t qtype, const void *W, const void *stage, float *y, float *slots,
                                           int *counters, int M, int N, int K, int dp_tiles, int pieces, int accum,
                                           hipStream_t s);
-int sera_mmq_group_tiles(int M, int count, const int *N);
-void sera_mmq_group_plan(int tiles, int M, int K, int cus, size_t max_slot_floats, int *dp_tiles, int *pieces);
+int sera_mmq_group_plan(int M, int count, const int *N, int K, int cus, size_t max_slot_floats, int *dp_tiles,
+                        int *pieces);
 hipError_t sera_launch_q4k_mmq_wide_group(uint32_t qtype, int count, const void *const *W, float *const *y,
                                           const int *N, const void *stage, float *slots, int *counters, int M, int K,
                                           int dp_tiles, int pieces, int accum, hipStream_t s);

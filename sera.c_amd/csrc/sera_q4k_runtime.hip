@@ -1259,11 +1259,10 @@ extern "C" int sera_linear_group(int count, const void *const *geometries, const
             if ((uintptr_t)outputs[i] < (uintptr_t)(outputs[j] + (size_t)M * N[j]) &&
                 (uintptr_t)outputs[j] < (uintptr_t)(outputs[i] + (size_t)M * N[i]))
                 disjoint = false;
-    const int group_tiles = q4 && disjoint && g_counters && g_cus > 0 ? sera_mmq_group_tiles(M, count, N) : 0;
-    if (group_tiles > 0) {
+    if (q4 && disjoint && g_counters && g_cus > 0) {
         int dp, pieces;
-        sera_mmq_group_plan(group_tiles, M, K, g_cus, partial_cap, &dp, &pieces);
-        if (pieces == 1 || group_tiles - dp <= kFewtokCounterBase) {
+        const int tiles = sera_mmq_group_plan(M, count, N, K, g_cus, partial_cap, &dp, &pieces);
+        if (tiles > 0 && (pieces == 1 || tiles - dp <= kFewtokCounterBase)) {
             if (sera_launch_q4k_mmq_wide_group(qt, count, weights, outputs, N, g_arena, partial, g_counters, M, K, dp,
                                                pieces, accum, s) != hipSuccess)
                 return fail(-3, "%s: grouped product launch failed", tag);

@@ -339,6 +339,27 @@ def test_prefill_tile_by_modelled_time(L):
     assert tiles64(386, 5644, 8192, cap=161 * 2 * 64 * 256) == 0 or pieces.value <= 2     # slots for two pieces
 
 
+def test_prefill_group_by_modelled_time(L):
+    """Groups over 64 tokens share a launch of 128 x 128 tiles unless their
+    padding to 128 tokens is modelled (and was measured) dearer than the
+    launches saved."""
+    dp, pieces = ctypes.c_int(), ctypes.c_int()
+
+    def plan(M, Ns, K):
+        tiles = L.sera_mmq_group_plan(M, len(Ns), (ctypes.c_int * len(Ns))(*Ns), K, 256, ctypes.c_size_t(1 << 30),
+                                      ctypes.byref(dp), ctypes.byref(pieces))
+        assert tiles in (0, -(-M // 128) * sum(-(-n // 128) for n in Ns))
+        return tiles
+
+    assert plan(512, [8192, 1024, 1024], 5120) and (dp.value, pieces.value) == (0, 3)
+    for M, Ns, K in ((512, [25600, 25600], 5120), (2048, [25600, 25600], 5120), (137, [21760, 21760], 768),
+                     (300, [4096, 1024, 1024, 132], 768)):
+        assert plan(M, Ns, K), (M, Ns, K)
+    for M, Ns, K in ((140, [42624, 42624], 512), (135, [42624, 42624], 2048), (64, [25600, 25600], 5120),
+                     (512, [25600], 5120), (512, [25600, 25602], 5120), (300, [1024, 1024], 2048)):
+        assert plan(M, Ns, K) == 0, (M, Ns, K)
+
+
 def test_kernel_launch_counts(L):
     """quantize + matmul (+ the split-K reduce when an MMQ launch splits K)."""
     assert L.sera_q4k_kernel_launches(1, 25600, 5120) == 2          # dot4 MMVQ
