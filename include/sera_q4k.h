@@ -177,6 +177,8 @@ int sera_q4k_mmq_splits(int M, int N, int K);
  * count) split the (tile, 256-wide K step) units evenly; split tiles are
  * summed in a fixed order by their last contributor, found with a per-tile
  * counter, so results repeat bit for bit and no workgroup waits on another.
+ * (On 128 x 128 tiles the full rounds of wgs tiles run whole and only the
+ * rest is split, as in the tail schedule below.)
  * slots: 2*wgs*sera_q4k_mmq_slot_floats(M) floats; counters:
  * sera_q4k_mmq_tiles(M, N) ints that must be zero and are zero again after
  * the kernel. Needs tiles*K/256 >= wgs. */

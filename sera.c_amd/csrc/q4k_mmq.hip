@@ -1110,70 +1110,6 @@ __global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_kernel(
     mmq_wide_store(sm, partial ? partial + (size_t)blockIdx.y * M * N : y, M, N, m0, n0, acc, partial ? 0 : accum);
 }
 
-/* Stream-K over wide tiles: the schedule and hand-off of
- * sera_q4k_mmq_streamk_kernel. */
-__global__ __launch_bounds__(256, 2) void sera_q4k_mmq_wide_streamk_kernel(
-        const uint8_t *__restrict__ W, const int8_t *__restrict__ xq, const uint32_t *__restrict__ xds,
-        float *__restrict__ y, float *__restrict__ slots, int *__restrict__ counters, int M, int Mpad, int N, int K,
-        int accum, int tiled) {
-    constexpr int NACC = 64;
-    __shared__ __attribute__((aligned(16))) MmqWideSmem<4> sm;
-    int &s_last = *(int *)&sm.sw[0][0][0];         /* a segment ends past a barrier */
-    const int tid = threadIdx.x;
-    const int P = gridDim.x;
-    const int w = (blockIdx.x & 7) * (P >> 3) + (blockIdx.x >> 3);
-    const int ntt = (M + kWideBM - 1) / kWideBM;
-    const int nrt = (N + kWideBN - 1) / kWideBN;
-    const int nkb = K / Q4K_QK;
-    const int64_t U = (int64_t)ntt * nrt * nkb;
-    const int64_t myu0 = sk_u0(w, U, P), myu1 = sk_u0(w + 1, U, P);
-    for (int64_t u = myu0; u < myu1;) {
-        const int t = (int)(u / nkb);
-        const int kb0 = (int)(u - (int64_t)t * nkb);
-        const int kb1 = (int)min<int64_t>(nkb, kb0 + (myu1 - u));
-        const int m0 = (t % ntt) * kWideBM, n0 = (t / ntt) * kWideBN;
-        v16f acc[4];
-        mmq_wide_tile(sm, W, xq, xds, Mpad, N, K, m0, n0, kb0, kb1, acc, tiled);
-        if (kb0 == 0 && kb1 == nkb) {
-            mmq_wide_store(sm, y, M, N, m0, n0, acc, accum);
-        } else {
-            const int64_t a = (int64_t)t * nkb;
-            const int c0 = sk_owner(a, U, P), c1 = sk_owner(a + nkb - 1, U, P);
-            float *mine = slots + (size_t)(2 * w + (myu0 <= a ? 1 : 0)) * (NACC * 256);
-#pragma unroll
-            for (int tt = 0; tt < 4; tt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    __hip_atomic_store(&mine[(size_t)(tt * 16 + r) * 256 + tid], acc[tt][r], __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            if (tid == 0)
-                s_last = __hip_atomic_fetch_add(&counters[t], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == c1 - c0;
-            __syncthreads();
-            const int last = s_last;
-            __syncthreads();                       /* read before the next tile writes sm */
-            if (last) {
-                if (tid == 0) __hip_atomic_store(&counters[t], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                for (int c = c0; c <= c1; c++) {
-                    const float *src = slots + (size_t)(2 * c + (sk_u0(c, U, P) <= a ? 1 : 0)) * (NACC * 256);
-#pragma unroll
-                    for (int tt = 0; tt < 4; tt++)
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const float v = __hip_atomic_load(&src[(size_t)(tt * 16 + r) * 256 + tid], __ATOMIC_RELAXED,
-                                                              __HIP_MEMORY_SCOPE_AGENT);
-                            acc[tt][r] = c == c0 ? v : acc[tt][r] + v;
-                        }
-                }
-                mmq_wide_store(sm, y, M, N, m0, n0, acc, accum);
-            }
-        }
-        __syncthreads();   /* the store may have used the activations' LDS */
-        u += kb1 - kb0;
-    }
-}
-
 /* Up to four matrices of one K on one activation stage: matrix i holds the
  * row tiles [end[i - 1], end[i]) of the launch. */
 struct MmqWideGroup {
@@ -1475,9 +1411,15 @@ extern "C" hipError_t sera_launch_q4k_mmq_streamk_acc(uint32_t qtype, const void
     if (sera_mmq_bm(M) == 32)
         return launch_mmq_streamk_cfg<1, 1, 4, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, P, accum, s);
     if (mmq_wide(M, N)) {
-        hipLaunchKernelGGL(sera_q4k_mmq_wide_streamk_kernel, dim3(P), dim3(256), 0, s, w, xq, xds, y, slots, counters,
-                           M, Mpad, N, K, accum, tiled);
-        return hipGetLastError();
+        /* 128 x 128 tiles: the full rounds of P whole, the R tiles left in as
+         * many K ranges as the slots hold, by the tail schedule's kernel (a
+         * persistent one spilled, and no call of the boundary reaches it) */
+        const int T = sera_mmq_tiles(M, N), R = T % P, nkb = K / Q4K_QK;
+        int pieces = R > 0 ? 2 * P / R : 1;
+        if (pieces > nkb) pieces = nkb;
+        if (pieces > 16) pieces = 16;
+        return sera_launch_q4k_mmq_wide_group(qtype, 1, &W, &y, &N, stage, slots, counters, M, K, T - R, pieces, accum,
+                                              s);
     }
     if (mmq_bn(M, N) == 128)
         return launch_mmq_streamk_cfg<1, 2, 2, 2>(tiled, w, xq, xds, y, slots, counters, M, N, K, P, accum, s);
