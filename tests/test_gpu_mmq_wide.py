@@ -1,8 +1,14 @@
 """The 128 x 128 MMQ tile (65 tokens and more on matrices of more than 64
-64 x 256 tiles, rows a multiple of 4) at the edges of its tiles: a last token tile of at most 64
-tokens, ragged rows, one to three K steps, every schedule, the accumulating
-and the unaligned store, both weight layouts. Exact inputs: every schedule
-must give the dequantized product bit for bit."""
+64 x 256 tiles, rows a multiple of 4) at the edges of its tiles: a last token
+tile of at most 64 tokens, ragged rows, one to sixteen K steps, every schedule,
+the accumulating and the unaligned store, both weight layouts; several matrices
+in one launch, whole and split along K; and the rules that choose between this
+tile and 64 x 256. On exact inputs (test_gpu_exact: one d8, one d) every
+schedule must give the dequantized product bit for bit; on random inputs, where
+each token and sub-block has its own scales, the product is the MMQ oracle's
+within 2e-5 * rms (the same terms in another order)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -30,8 +36,6 @@ def test_wide_tile_exact(torch, M, N, K):  # noqa: F811
         layouts.append((q3q4.QTYPE_Q4K_TILED, dev(torch, q3q4.q4k_tiled_bytes(W, N, K))))
     for qt, Wd in layouts:
         for s in sorted({1, nkb}):
-            if s > 1 and M * N % 4:
-                continue
             say(f"case wide plain qt={qt} M={M} N={N} K={K} splits={s}")
             y = nan_out(torch, M, N)
             part = torch.empty(s * M * N, dtype=torch.float32, device="cuda") if s > 1 else None
@@ -68,6 +72,127 @@ def test_wide_tile_exact(torch, M, N, K):  # noqa: F811
     assert float(buf[0]) == -7.0 and float(buf[-1]) == -7.0, "store past Y"
 
 
+def random_inputs(rng, M, K, rows):
+    """Activations with outlier channels, and Q4_K rows."""
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    X[:, rng.choice(K, K // 100, replace=False)] *= 20.0
+    return X, [oracle.quantize_q4k((rng.standard_normal((n, K)) * 0.02).astype(np.float32)) for n in rows]
+
+
+def assert_oracle(y, W, q, what):
+    """Sampled rows (the first and last tiles' among them) of y, all tokens,
+    against the MMQ oracle on the staged activations q = (quants, d8, s8)."""
+    N, K = W.shape[0], q[0].shape[1]
+    rows = np.unique(np.r_[0:4, N - 20:N, np.linspace(0, N - 1, 60).astype(int)])
+    ref = oracle.gemm_mmq(W[rows], *q, len(rows), K)
+    err = float(np.max(np.abs(y[:, rows].astype(np.float64) - ref)) / np.sqrt(np.mean(ref * ref)))
+    say(f"  {what}: max|err| / rms = {err:.2e}")
+    assert np.all(np.isfinite(y)) and err <= 2e-5, what
+
+
+# M % 128 in 1..64: the 64-token body beside the 128-token one (192: as its only second tile); rows a multiple of 16 that
+# do not fill a tile, both layouts; eight and sixteen K steps; whole, all split, one tile split
+@pytest.mark.parametrize("M,N,K", [(129, 5648, 2304), (192, 5636, 2048), (577, 2064, 4096)])
+def test_wide_tile_scales(torch, M, N, K):  # noqa: F811
+    tiles = -(-M // 128) * -(-N // 128)
+    assert q3q4.load().sera_q4k_mmq_tiles(M, N) == tiles, "not a wide-tile case"
+    X, (W,) = random_inputs(np.random.default_rng(M + N + K), M, K, [N])
+    W = W.reshape(N, -1)
+    q, st = oracle.q8_1_mmq(X), mmq_stage(torch, X)
+    layouts = [(12, dev(torch, W))]
+    if N % 16 == 0:
+        layouts.append((q3q4.QTYPE_Q4K_TILED, dev(torch, q3q4.q4k_tiled_bytes(W, N, K))))
+    for qt, Wd in layouts:
+        for dp, pieces in ((tiles, 1), (0, 3), (tiles - 1, K // 256)):
+            say(f"case wide scales qt={qt} M={M} N={N} K={K} dp_tiles={dp} pieces={pieces}")
+            slots = torch.empty(max(q3q4.mmq_tail_slot_floats(M, N, dp, pieces), 1), dtype=torch.float32, device="cuda")
+            counters = torch.zeros(max(tiles - dp, 1), dtype=torch.int32, device="cuda")
+            y = nan_out(torch, M, N)
+            q3q4.mmq_tail(Wd, st, y, M, N, K, dp, pieces, slots=slots, counters=counters, qtype=qt)
+            torch.cuda.synchronize()
+            assert int(counters.abs().sum()) == 0, "tile counters not reset"
+            assert_oracle(y.cpu().numpy(), W, q, f"dp_tiles={dp} pieces={pieces}")
+
+
+# all tiles split along K, and whole rounds before a split tail; a matrix whose last row tile is ragged between others
+@pytest.mark.parametrize("M,Ns,K", [(129, [4096, 1024, 528], 2560), (193, [4096, 1040, 528, 64], 4096),
+                                    (577, [7168, 6400], 2304)])
+def test_group_split_along_k(torch, M, Ns, K):  # noqa: F811
+    """A grouped launch whose plan has several pieces: every matrix against the
+    oracle, plain, with RMSNorm, on tiles, accumulating (product + add bit for
+    bit), into outputs that are only 4-byte aligned, replayed from a graph
+    between eager calls, and whole where the arena has no room for slots."""
+    L = q3q4.load()
+    lin = q3q4.Linear(device=0, max_tokens=640, max_features=8192, max_k=4096)
+    dp, pieces = ctypes.c_int(), ctypes.c_int()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tiles = L.sera_mmq_group_plan(M, len(Ns), (ctypes.c_int * len(Ns))(*Ns), K, cus, ctypes.c_size_t(1 << 25),
+                                  ctypes.byref(dp), ctypes.byref(pieces))
+    assert tiles == -(-M // 128) * sum(-(-n // 128) for n in Ns) and pieces.value > 1 and (dp.value > 0) == (M == 577)
+    rng = np.random.default_rng(M + sum(Ns) + K)
+    X, Ws = random_inputs(rng, M, K, Ns)
+    Ws = [w.reshape(n, -1) for w, n in zip(Ws, Ns)]
+    Xd, Wd, geos = dev(torch, X), [dev(torch, w) for w in Ws], [q3q4.bind_geometry(12, K, n) for n in Ns]
+    say(f"case group split M={M} Ns={Ns} K={K} dp_tiles={dp.value} of {tiles} pieces={pieces.value}")
+
+    def run(ys, **kw):
+        q3q4.linear_group(kw.pop("geos", geos), kw.pop("W", Wd), ys, Xd, **kw)
+        torch.cuda.synchronize()
+        assert int(lin.workspace[:256 << 10].to(torch.int32).abs().sum()) == 0, "counters not reset"
+        return ys
+
+    q = oracle.q8_1_mmq(X)
+    plain = run([nan_out(torch, M, n) for n in Ns])
+    for y, w in zip(plain, Ws):
+        assert_oracle(y.cpu().numpy(), w, q, "plain")
+    gamma = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    qn = oracle.q8_1_mmq(oracle.rmsnorm_fused_order(X, gamma, 1e-6))
+    for y, w in zip(run([nan_out(torch, M, n) for n in Ns], gamma=dev(torch, gamma), eps=1e-6, flags=q3q4.LIN_RMSNORM), Ws):
+        assert_oracle(y.cpu().numpy(), w, qn, "RMSNorm")
+    tiled = run([nan_out(torch, M, n) for n in Ns], geos=[q3q4.bind_geometry(q3q4.QTYPE_Q4K_TILED, K, n) for n in Ns],
+                W=[dev(torch, q3q4.q4k_tiled_bytes(w, n, K)) for w, n in zip(Ws, Ns)])
+    base = [torch.randn((M, n), device="cuda") for n in Ns]
+    acc = run([b.clone() for b in base], flags=q3q4.LIN_ACCUMULATE)
+    bufs = [torch.full((M * n + 1,), -7.0, device="cuda") for n in Ns]
+    odd = run([b[1:].view(M, n) for b, n in zip(bufs, Ns)])
+    for i in range(len(Ns)):
+        assert torch.equal(tiled[i], plain[i]) and torch.equal(odd[i], plain[i]) and float(bufs[i][0]) == -7.0
+        assert torch.equal(acc[i], base[i] + plain[i])
+    ys = [torch.zeros((M, n), device="cuda") for n in Ns]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q3q4.linear_group(geos, Wd, ys, Xd)
+    for _ in range(3):
+        for y in ys:
+            y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(ys, plain)), "replay differs"
+        run([nan_out(torch, M, n) for n in Ns])
+    stage = q3q4.mmq_stage_layout(M, K)["total"]
+    small = torch.zeros((256 << 10) + stage, dtype=torch.uint8, device="cuda")
+    assert L.sera_q4k_set_arena(ctypes.c_void_p(small.data_ptr()), small.numel()) == 0
+    ys = [nan_out(torch, M, n) for n in Ns]
+    q3q4.linear_group(geos, Wd, ys, Xd)
+    torch.cuda.synchronize()
+    for y, w in zip(ys, Ws):
+        assert_oracle(y.cpu().numpy(), w, q, "no slots")
+    q3q4.Linear(device=0, max_tokens=640, max_features=8192, max_k=4096)
+
+
+# few enough 128 x 128 tiles for split-K where the 64 x 256 ones would be too many for it
+@pytest.mark.parametrize("M,N,K", [(330, 2640, 1024), (1100, 832, 768)])
+def test_split_k_on_wide_tiles(torch, M, N, K):  # noqa: F811
+    lin = q3q4.Linear(device=0, max_tokens=1152, max_features=2688, max_k=1024)
+    assert q3q4.load().sera_q4k_mmq_tiles(M, N) <= 64 and q3q4.load().sera_q4k_mmq_schedule(M, N, K) == 0
+    W, X = exact_inputs(np.random.default_rng(M + N), M, N, K)
+    say(f"case split-K on wide tiles M={M} N={N} K={K} splits={q3q4.mmq_splits(M, N, K)}")
+    y = nan_out(torch, M, N)
+    lin(q3q4.bind_geometry(12, K, N), dev(torch, W), dev(torch, X), y)
+    torch.cuda.synchronize()
+    assert_bits(y, expected(W, X, N, K), "boundary")
+
+
 @pytest.mark.parametrize("M,Ns,K", [(65, [8192, 512, 260], 512), (200, [4096, 1024, 1024, 132], 768),
                                     (129, [3000, 3000], 256), (300, [1024, 1024], 2048)])
 def test_group_in_one_launch(torch, M, Ns, K):  # noqa: F811
@@ -94,7 +219,7 @@ def test_group_in_one_launch(torch, M, Ns, K):  # noqa: F811
     assert lin.workspace_bytes > 0
 
 
-# M * N % 4 != 0: no split-K, so the tail schedule cuts the tiles along K
+# M * N % 4 != 0: no split-K, so the tail schedule runs them, cut along K where that is modelled faster
 @pytest.mark.parametrize("M,N,K", [(203, 1333, 1792), (41, 1333, 1024), (19, 3001, 2048), (13, 1001, 2304), (65, 77, 256)])
 def test_odd_products_split_by_the_tail(torch, M, N, K):  # noqa: F811
     L = q3q4.load()
