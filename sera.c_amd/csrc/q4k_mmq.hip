@@ -457,8 +457,13 @@ __device__ __forceinline__ void mmq_segment(
 
 /* Store an output tile: lane holds weight row n0+64*wn+32*nt+l32 for tokens
  * m0+BMW*wt+32*t + 8*(r/4) + 4*h + r%4 (paired tile: r < 8, the sum of the
- * even and odd sub-block rows r and r + 8). */
-template <int TT, int WGT, int WGN, int PR = 0>
+ * even and odd sub-block rows r and r + 8). ATONCE: an accumulating store has
+ * a row tile's loads and sums before its first store; load, add and store in
+ * turn wait for each load (us a call, accumulating: 6704 x 1024 at 565 tokens
+ * 36.6 -> 26.2, 25600 x 5120 at 37 48.9 -> 42.0). The stream-K kernels store
+ * in turn: their segment loop has no registers to spare (151936 x 5120 at 24
+ * tokens 141.9 us, at once 148.4). */
+template <int TT, int WGT, int WGN, int PR = 0, bool ATONCE = true>
 __device__ __forceinline__ void mmq_store(float *__restrict__ out, int M, int N, int m0, int n0,
                                           const v16f (&acc)[TT][2], int accum) {
     constexpr int BMW = MmqShape<TT, WGT, WGN, PR>::BMW;
@@ -472,14 +477,23 @@ __device__ __forceinline__ void mmq_store(float *__restrict__ out, int M, int N,
 #pragma unroll
         for (int t = 0; t < TT; t++) {
             constexpr int NR = PR ? 8 : 16;
+            if constexpr (!ATONCE) {
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    const int m = m0 + BMW * wt + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
+                    const float v = PR ? acc[t][nt][r] + acc[t][nt][r + 8] : acc[t][nt][r];
+                    if (m < M) {
+                        float *dst = out + (size_t)m * N + n;
+                        *dst = accum ? *dst + v : v;
+                    }
+                }
+                continue;
+            }
             const int mb = m0 + BMW * wt + 32 * t + 4 * h;      /* row r: mb + 8 * (r / 4) + r % 4 */
             float *dst = out + (size_t)mb * N + n;
             float v[NR];
 #pragma unroll
             for (int r = 0; r < NR; r++) v[r] = PR ? acc[t][nt][r] + acc[t][nt][r + 8] : acc[t][nt][r];
-            /* all loads before the first store: load, add and store in turn
-             * waited for each load (us a call, accumulating: 6704 x 1024 at
-             * 565 tokens 36.6 -> 26.2, 25600 x 5120 at 37 48.9 -> 42.0) */
             if (accum) {
                 float o[NR];
 #pragma unroll
@@ -559,7 +573,7 @@ __global__ __launch_bounds__(256, WPE) void sera_q4k_mmq_streamk_kernel(
         v16f acc[TT][2];
         mmq_segment<TT, WGT, WGN, PR, TT == 1 && WPE <= 2>(sm, W, xq, xds, N, K, m0, n0, kb0, kb1, acc, tiled);
         if (kb0 == 0 && kb1 == nkb) {
-            mmq_store<TT, WGT, WGN, PR>(y, M, N, m0, n0, acc, accum);
+            mmq_store<TT, WGT, WGN, PR, false>(y, M, N, m0, n0, acc, accum);
         } else {
             /* slot rule: 2c for a contributor c whose range starts inside the
              * tile, 2c + 1 for one that started before it (then the tile is
@@ -600,7 +614,7 @@ __global__ __launch_bounds__(256, WPE) void sera_q4k_mmq_streamk_kernel(
                                 acc[tt][nt][r] = c == c0 ? v : acc[tt][nt][r] + v;
                             }
                 }
-                mmq_store<TT, WGT, WGN, PR>(y, M, N, m0, n0, acc, accum);
+                mmq_store<TT, WGT, WGN, PR, false>(y, M, N, m0, n0, acc, accum);
             }
         }
         u += kb1 - kb0;
