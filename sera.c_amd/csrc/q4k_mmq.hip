@@ -15,7 +15,8 @@
  *     columns = weight rows), so in the 32x32 result each lane owns one
  *     weight row: its sub-block scale fp16(d*sc_b) is a per-lane value the
  *     lane decodes from the block header it loaded itself, and the token
- *     scales d8 come from LDS as float4s.
+ *     scales d8 come from LDS as float4s. (The 128 x 128 tile has the two
+ *     operands the other way round; see there.)
  *   - the fp32 epilogue is two VALU ops per element and sub-block, with no
  *     int-to-float convert: the MFMA's int32 accumulator starts at the bit
  *     pattern of 1.5 * 2^23, so its result, read as a float, is exactly
@@ -37,8 +38,8 @@
  *     super-block by one v_mfma_f32_32x32x16_f16 accumulating into the same
  *     fp32 tile (fp16 x fp16 products are exact in fp32).
  *   - activations (int8 quants, d8, s8) for the workgroup's tokens are
- *     staged in LDS, double buffered per 256-wide K step, rows padded to
- *     272 bytes so 16 consecutive tokens' 16-byte reads hit distinct banks.
+ *     staged in LDS, double buffered per 256-wide K step, columns swizzled
+ *     so 16 consecutive tokens' 16-byte reads hit distinct banks.
  *     Weights are not staged: each lane loads its row's 16-byte nibble
  *     pieces straight into registers (16 consecutive int8 of one row is the
  *     B operand) and unpacks them in registers; one piece feeds the two
@@ -411,8 +412,9 @@ __device__ __forceinline__ void mmq_segment(
                  * element are plain fp32 instructions, four of the first kind
                  * before the four that use them: with two waves per SIMD they
                  * issue every 2.3-2.6 cycles against 4.4 for v_fma_mix on fp16
-                 * scales (gate/up 25600 x 5120 at 512 tokens 209 -> 197 us,
-                 * 2048 tokens 752 -> 695, down 217 -> 198, same results), for
+                 * scales (us a call: gate/up 25600 x 5120 at 512 tokens 202.9
+                 * -> 193.0, 2048 tokens 831 -> 732, down at 512 219.3 ->
+                 * 193.0, same results), for
                  * four LDS reads per (sub-block, token tile) instead of two. */
                 const float *d8p = &sm.d8[buf][b][BMW * wt + 32 * t + 16 * h];
 #pragma unroll
@@ -715,7 +717,7 @@ __global__ __launch_bounds__(256, WPE) void sera_q4k_mmq_tail_kernel(
 
 /* ---- wide tile: 128 tokens x 128 rows --------------------------------------- */
 
-/* Prefill tile for more than 64 tokens (sera_mmq_wide): four waves of 128
+/* Prefill tile for more than 64 tokens (mmq_wide): four waves of 128
  * tokens x 32 rows. Weights are the MFMA's A operand here (result rows =
  * weight rows) and activations its B operand (a lane owns one token), so
  *   - a wave unpacks its 32 rows once for four token tiles (the 64 x 256 tile
@@ -733,8 +735,8 @@ __global__ __launch_bounds__(256, WPE) void sera_q4k_mmq_tail_kernel(
  * the epilogue of unit i; the one barrier of a step comes three units before
  * its end and waits for loads issued most of a step earlier. Cycles per
  * launch at 2048 tokens of gate/up (25600 x 5120): 1.66M with the 64 x 256
- * tile at half-rate FMAs, 1.42M at full rate, 1.25M here; 752 -> 695 -> 675
- * us. Issuing all activation loads at once costs 5% (the wave waits for the
+ * tile at half-rate FMAs, 1.42M at full rate, 1.25M here; 831 -> 732 -> 677
+ * us a call. Issuing all activation loads at once costs 5% (the wave waits for the
  * queue), two waves per SIMD of one 8-wave workgroup was not tried, and
  * reading the activations three or five units ahead instead of two is within
  * 1%.
@@ -1241,13 +1243,11 @@ extern "C" hipError_t sera_launch_splitk_reduce(const float *partial, float *y, 
 
 /* Token-tile width of the workgroup for M tokens: 16 (the paired tile, one
  * per wave), 32 (one token tile per wave, 4 waves along weight rows) or 64
- * (two per wave); all at 2 waves per SIMD, and all tiles span 256 weight
- * rows. The 32-token tile ran at 3 waves per SIMD until the magic-seeded
- * epilogue: its 16 seed registers made that budget spill (37 -> 52 us on
- * gate/up at 32 tokens), while at 2 waves with the next step's weights
- * issued ahead it measures 37 us. Measured on MI355X against 128 x
- * 128 tiles (both under stream-K): the 64 x 256 tile is the fastest at 512
- * tokens for both the 5120 -> 25600 and the 25600 -> 5120 shapes. */
+ * (two per wave), all at 2 waves per SIMD and, but for the 64 x 128 and 128 x
+ * 128 tiles below, of 256 weight rows. The 32-token tile ran at 3 waves per
+ * SIMD until the magic-seeded epilogue: its 16 seed registers made that budget
+ * spill (37 -> 52 us on gate/up at 32 tokens), while at 2 waves with the next
+ * step's weights issued ahead it measures 37 us. */
 extern "C" int sera_mmq_bm(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : 64; }
 
 /* Weight rows per tile: 256, or 128 for the 64-token tile when 256-row
@@ -1266,16 +1266,17 @@ static int mmq_bn(int M, int N) {
     return 256;
 }
 
-/* Whether M tokens of an N-row matrix run the 128 x 128 wide tile: from 65
- * tokens wherever the 64-token tile would take 256 rows. On one MI355X, us
- * against the 64 x 256 tile (both with the tail schedule and full-rate FMAs):
- * gate/up at 96 / 256 / 512 / 2048 tokens 65.2 / 123.1 / 191.3 / 675 against
- * 69.9 / 125.0 / 197.8 / 714, down at 512 186.5 against 194.5, o at 256 47.8
- * against 50.2, q at 512 70.9 against 72.3. The narrow matrices keep the
- * 64 x 128 tile, which leaves them twice as many tiles. Rows of Y that are
- * not 16-byte aligned keep the 64 x 256 tile: its lanes hold neighbouring
- * rows, the wide tile's go through LDS, which a short K does not pay for
- * (6706 x 512 at 565 tokens 17.3 against 20.3 us). */
+/* Whether the tiles of M tokens of an N-row matrix are the 128 x 128 wide
+ * ones: from 65 tokens wherever the 64-token tile would take 256 rows; the
+ * boundary still takes 64 x 256 where sera_mmq_plan64 says so. On one MI355X,
+ * us a call, 64 x 256 / wide (both with the tail schedule and full-rate FMAs):
+ * gate/up 25600 x 5120 at 128 / 512 / 2048 tokens 66.6 / 63.2, 193.0 / 185.7,
+ * 732 / 677, down 5120 x 25600 at 512 / 2048 193.0 / 185.3, 762 / 698, q 8192
+ * x 5120 at 512 74.5 / 72.2. The narrow matrices keep the 64 x 128 tile, which
+ * leaves them twice as many tiles. Rows of Y that are not 16-byte aligned keep
+ * the 64 x 256 tile: its lanes hold neighbouring rows, the wide tile's go
+ * through LDS, which a short K does not pay for (6706 x 512 at 565 tokens 17.3
+ * against 20.3 us). */
 static int mmq_wide(int M, int N) { return M > 64 && N % 4 == 0 && mmq_bn(M, N) == 256; }
 
 /* Output tiles of the MMQ grid for M tokens. */
@@ -1469,14 +1470,19 @@ static const sera_tile_cost &tile_cost(int M, int N) {
  * least modelled time, which it returns. The device keeps 2 workgroups per CU resident, so P =
  * 2 * cus run per round. The whole tiles are a multiple of P (all full
  * rounds, or one round fewer); the R tiles left are cut into c K ranges (c =
- * 1: whole as well). The split tiles' slots must fit max_slot_floats. */
+ * 1: whole as well), where that is modelled to save 1%: after many full rounds
+ * the ends are staggered and less gives nothing (6400 tiles of 20 super-blocks,
+ * the last half round whole 1330 us a call, in two ranges 1344). The split
+ * tiles' slots must fit max_slot_floats. */
+static constexpr float kSplitGain = 0.99f;
 static float tail_plan(const sera_tile_cost &k, int T, int nkb, int cus, size_t slot_floats, size_t max_slot_floats,
                        int *dp_tiles, int *pieces) {
     const int C = cus > 0 ? cus : kModelCUs;
     const int P = 2 * C;
     const int rounds = T / P;
     int best_dp = T, best_c = 1;
-    float best = sera_plan_cost(&k, rounds, T - (long)rounds * P, 1, nkb, C);
+    const float whole = sera_plan_cost(&k, rounds, T - (long)rounds * P, 1, nkb, C);
+    float best = kSplitGain * whole;
     for (int fold = 0; fold <= (rounds > 0 ? 1 : 0); fold++) {
         const int dp = (rounds - fold) * P;
         const int R = T - dp;
@@ -1489,7 +1495,7 @@ static float tail_plan(const sera_tile_cost &k, int T, int nkb, int cus, size_t 
     }
     *dp_tiles = best_dp;
     *pieces = best_c;
-    return best;
+    return best_c == 1 ? whole : best;
 }
 
 extern "C" void sera_mmq_tail_plan(int M, int N, int K, int cus, size_t max_slot_floats, int *dp_tiles,

@@ -422,10 +422,11 @@ bool use_streamk(int M, int N, int K) { return g_counters && streamk_rule(M, N, 
  * tiles the tail won: o at 256 tokens 50.6 against 54.4, gate/up at 64
  * 44.1 against 48.8, at 512 215.9 against 232.9, down at 512 206.5 against
  * 217.9). It also serves, at any batch (below a full round of 16- or
- * 32-token tiles), the products whose M*N is no multiple of 4, which split-K's 16-byte reduce cannot: run whole, their few
- * tiles left most CUs idle (1333 x 1792 at 203 tokens, 44 tiles: 21.7 us
- * whole, 12 in 4 pieces). Its counters share the stream-K half of the counter
- * region (the two never run at once; both leave it zero). */
+ * 32-token tiles), the products whose M*N is no multiple of 4, which split-K's
+ * 16-byte reduce cannot: run whole, their few tiles leave most CUs idle on a
+ * long K (1333 x 1792 at 203 tokens, 44 tiles: 24.1 us a call whole, 15.8 in
+ * pieces). Its counters share the stream-K half of the counter region (the two
+ * never run at once; both leave it zero). */
 bool tail_rule(int M, int N) {
     if (g_cus <= 0) return false;
     if (((size_t)M * N) % 4 != 0) return sera_mmq_bm(M) == 64 || sera_mmq_tiles(M, N) < streamk_wgs(M);

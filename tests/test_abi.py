@@ -352,6 +352,7 @@ def test_prefill_group_by_modelled_time(L):
         return tiles
 
     assert plan(512, [8192, 1024, 1024], 5120) and (dp.value, pieces.value) == (0, 3)
+    assert plan(2048, [25600, 25600], 5120) == 6400 and (dp.value, pieces.value) == (6400, 1)   # half a round: not worth it
     for M, Ns, K in ((512, [25600, 25600], 5120), (2048, [25600, 25600], 5120), (137, [21760, 21760], 768),
                      (300, [4096, 1024, 1024, 132], 768)):
         assert plan(M, Ns, K), (M, Ns, K)
