@@ -414,8 +414,8 @@ __device__ __forceinline__ void mmq_segment(
                  * issue every 2.3-2.6 cycles against 4.4 for v_fma_mix on fp16
                  * scales (us a call: gate/up 25600 x 5120 at 512 tokens 202.9
                  * -> 193.0, 2048 tokens 831 -> 732, down at 512 219.3 ->
-                 * 193.0, same results), for
-                 * four LDS reads per (sub-block, token tile) instead of two. */
+                 * 193.0, same results), for four LDS reads per (sub-block,
+                 * token tile) instead of two. */
                 const float *d8p = &sm.d8[buf][b][BMW * wt + 32 * t + 16 * h];
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
